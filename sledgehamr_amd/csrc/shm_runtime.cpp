@@ -897,21 +897,162 @@ void Runtime::fill_params(double *blk, double time, double dt, double dx,
 LaunchCfg Runtime::resolved_launch(int lev) const {
     const LaunchCfg t = lev + 1 >= 0 && lev + 1 < (int)tuned_.size() ? tuned_[lev + 1]
                                                                      : LaunchCfg();
-    auto pick = [](int user, int tuned, int dflt) {
-        return user >= 0 ? user : (tuned >= 0 ? tuned : dflt);
+    const LevelState *ls = lev == -1 ? (shadow_.defined() ? &shadow_ : nullptr)
+                           : has_level(lev) ? &levels_[lev] : nullptr;
+    // The size rule fills in where neither the caller nor the autotuner has
+    // fixed a tile shape or chunk length.
+    LaunchCfg r;
+    if (ls && launch.variant < 0 && launch.tz == 0 && t.variant < 0) {
+        LaunchCfg &c = ls->rule[launch.fused < 0 ? 0 : launch.fused ? 2 : 1];
+        if (c.variant < 0) c = rule_launch(*ls, launch.fused);
+        r = c;
+    }
+    auto pick = [](int user, int tuned, int rule, int dflt) {
+        return user >= 0 ? user : tuned >= 0 ? tuned : rule >= 0 ? rule : dflt;
     };
     LaunchCfg c;
-    c.variant = pick(launch.variant, t.variant, kDefaultVariant);
-    c.tz = launch.tz > 0 ? launch.tz : t.tz;
-    c.xcd_split = pick(launch.xcd_split, t.xcd_split, 1);
-    c.persistent = pick(launch.persistent, t.persistent, 1);
-    c.zc_minor = pick(launch.zc_minor, t.zc_minor, 0);
-    c.fused = pick(launch.fused, t.fused, 0);
+    c.variant = pick(launch.variant, t.variant, r.variant, kDefaultVariant);
+    c.tz = launch.tz > 0 ? launch.tz : t.tz > 0 ? t.tz : r.tz;
+    c.xcd_split = pick(launch.xcd_split, t.xcd_split, -1, 1);
+    c.persistent = pick(launch.persistent, t.persistent, -1, 1);
+    c.zc_minor = pick(launch.zc_minor, t.zc_minor, -1, 0);
+    c.fused = pick(launch.fused, t.fused, r.fused, 0);
     int dv = -1;
     const FusedEntry *row = fused_row();
     for (int v = kNVar - 1; v >= 0 && dv < 0; --v)
         if (row[v].fn) dv = v;
-    c.fused_variant = pick(launch.fused_variant, t.fused_variant, dv);
+    c.fused_variant = pick(launch.fused_variant, t.fused_variant, r.fused_variant, dv);
+    return c;
+}
+
+/** The launch shape the box sizes ask for.  A stage kernel's time is modelled
+ *  as the planes a resident workgroup walks one after the other (rounds of
+ *  the grid times the chunk with its R extra queue planes), plus a small
+ *  share for the wavefront planes of the whole grid; constants fitted to a
+ *  sweep of every shape over 32^3..320^3 levels of one and two fields in
+ *  three precisions, where the pick is within 2 % of the fastest shape on
+ *  average (default shape 64 x 8 with 16-plane chunks: 25 % on average, 1.55x
+ *  at 32^3, where its 4 workgroups walk 16 planes each). */
+LaunchCfg Runtime::rule_launch(const LevelState &ls, int fused) const {
+    LaunchCfg c;
+    c.variant = kDefaultVariant;
+    c.fused = 0;
+    const auto &boxes = ls.L.boxes;
+    // GW levels run as component groups and dissipation is built for one
+    // tile shape: the default with its automatic chunk length is within 1 %
+    // of the autotuner's pick there (384^3: 6.74 against 6.69 ms).
+    if (gw_ || ko_ || boxes.empty()) return c;
+    const int kind = integrator_ == 10 ? kSsprk1 : integrator_ == 11 ? kLeap1 : kRkn0;
+    const auto &row = kt_.stage[kind][(int)prec_][R_][0][0];
+    int maxn = 1;
+    for (const Box3 &b : boxes) maxn = std::max(maxn, b.n(2));
+    const bool one_field = kt_.nfields == 1 && !tile_lo();
+    auto usable = [&](int v) {
+        if (!row[v].fn) return false;
+        // Two rows per thread pay where a thread holds one short queue (one
+        // stencil component read as stored: 255 against 315 us at 256^3)
+        // and cost registers elsewhere (519 against 470 us with two).
+        if (kVariants[v].ry > 1) return one_field;
+        if (one_field && kVariants[v].tx == 64 && kVariants[v].nw > 4) return false;
+        // At radius 3 a 32 x 8 tile's ring has more cells than the tile.
+        return kVariants[v].tx == 64 || R_ < 3;
+    };
+    auto tiles = [&](int tx, int ty, int z, double &planes) {
+        long long n = 0;
+        planes = 0;
+        for (const Box3 &b : boxes) {
+            const long long xy = (long long)((b.n(0) + tx - 1) / tx) * ((b.n(1) + ty - 1) / ty);
+            const int k = (b.n(2) + z - 1) / z;
+            n += xy * k;
+            planes += (double)xy * (b.n(2) + k * R_);
+        }
+        return n;
+    };
+    auto cost = [&](int v, int z) {
+        double planes;
+        const TileVariant &t = kVariants[v];
+        const long long n = tiles(t.tx, t.nw * 64 / t.tx * t.ry, z, planes);
+        const long long slots = (long long)ncu_ * std::max(1, 12 / t.nw);
+        return (double)((n + slots - 1) / slots) * (z + R_) +
+               0.03 * planes * t.nw * t.ry / ncu_;
+    };
+    auto best_variant = [&](int z) {
+        int bv = -1;
+        for (int v = 0; v < kNVar; ++v)
+            if (usable(v) && (bv < 0 || cost(v, z) < cost(bv, z))) bv = v;
+        return bv;
+    };
+    // Fused first two stages: one workgroup per CU, a chunk costs 3R + 2
+    // extra planes.  SSPRK3 on tiles of the stored type: 354 against 469 us
+    // at 256^3 (FP32 + bf16), 576 against 805 us (FP64); 97 to 81 us at
+    // 128^3.  RKN: FP64 up to radius 2 only (340 against 382 us at 256^3;
+    // FP32 within 2 % either way, radius 3 slower).  FP64 tiles of stored
+    // pairs, and ensembles (1.57 against 1.42 ms for 64 boxes): slower.
+    const bool pays = boxes.size() == 1 && maxn >= 64 && !tile_lo() &&
+                      (integrator_ == 10 || (prec_ == Prec::F64 && R_ <= 2));
+    if (fused != 0 && fused_possible(ls) && (fused > 0 || pays)) {
+        const FusedEntry *frow = fused_row();
+        double bc = 1e30;
+        int bv = -1, bz = maxn;
+        // The widest tile that still gives half the CUs work at 8 planes.
+        for (int v = kNVar - 1; v >= 0; --v) {
+            double p;
+            if (!frow[v].fn) continue;
+            if (bv < 0 || tiles(64, frow[bv].ty, std::min(8, maxn), p) < ncu_ / 2) bv = v;
+        }
+        for (int k = 1; k <= maxn; ++k) {
+            const int z = (maxn + k - 1) / k;
+            if (z < 4 && k > 1) break;
+            double p;
+            const long long n = tiles(64, frow[bv].ty, z, p);
+            const double m = (double)((n + ncu_ - 1) / ncu_) * (z + 3 * R_ + 2);
+            if (m < bc) {
+                bc = m;
+                bz = z;
+            }
+        }
+        c.fused = 1;
+        c.fused_variant = bv;
+        c.tz = bz;
+        c.variant = best_variant(bz);
+        return c;
+    }
+    if (boxes.size() == 1) {
+        double bc = 1e30;
+        for (int z = 4; z < 2 * maxn; z *= 2) {
+            const int zz = std::min(z, maxn), v = best_variant(zz);
+            if (cost(v, zz) < bc) {
+                bc = cost(v, zz);
+                c.variant = v;
+                c.tz = zz;
+            }
+        }
+        return c;
+    }
+    // Many boxes: enough tiles that the rounds even out, so the shape with
+    // the least padding wins (measured weight per padded cell: a 32-wide
+    // plane 1.2x a 64-wide one; 16..64-cell boxes: 2.95 to 2.37 ms for the
+    // three SSPRK3 stages of 39.5 M cells, 32^3..160^3: 1.62 to 1.50 ms per
+    // RKN4 step with two rows per thread), on chunks of 16 planes, or 8
+    // where 16 leave fewer than four tiles per CU.
+    double bw = 1e30;
+    for (int v = 0; v < kNVar; ++v) {
+        if (!usable(v)) continue;
+        const TileVariant &t = kVariants[v];
+        double planes;
+        (void)tiles(t.tx, t.nw * 64 / t.tx * t.ry, std::min(16, maxn), planes);
+        const double w = planes * t.nw * t.ry *
+                         (t.tx == 32 ? 1.2 : t.nw == 4 && t.ry == 1 ? 1.1 : t.nw == 16 ? 1.05 : 1.);
+        if (w < bw) {
+            bw = w;
+            c.variant = v;
+        }
+    }
+    const TileVariant &t = kVariants[c.variant];
+    double p;
+    c.tz = 16;
+    while (c.tz > 4 && tiles(t.tx, t.nw * 64 / t.tx * t.ry, c.tz, p) < 4LL * ncu_) c.tz /= 2;
+    c.tz = std::min(c.tz, maxn);
     return c;
 }
 

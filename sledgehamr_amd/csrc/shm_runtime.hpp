@@ -103,6 +103,18 @@ struct Layout {
     long long nvalid() const { return vprefix.empty() ? 0 : vprefix.back(); }
 };
 
+/** Launch shape of the stage kernels.  A field of -1 (tz: 0) is not set: the
+ *  level's tuned value, else the size rule (Runtime::rule_launch) applies. */
+struct LaunchCfg {
+    int variant = -1;     // tile shape index into kVariants
+    int tz = 0;           // z-chunk length of a tile (0: automatic)
+    int xcd_split = -1;   // each XCD walks one contiguous range of tiles
+    int persistent = -1;  // grid = resident capacity (1) or one tile per workgroup (0)
+    int zc_minor = -1;    // tile order: z-chunk outermost (0) or innermost (1)
+    int fused = -1;       // SSPRK3 stages one and two in one launch (0/1)
+    int fused_variant = -1;  // tile shape of that launch
+};
+
 /** Device state of one level: the old/new state pair and stage scratch. */
 struct LevelState {
     Layout L;
@@ -150,6 +162,9 @@ struct LevelState {
     int mnseg_in = 0, mnseg_out = 0;
     long long mtot_in = 0, mtot_out = 0;
     long mirror_epoch = -1;
+    // Launch shapes of the size rule, by what is asked about fusing the
+    // first two stages (not asked, off, on); variant -1: not computed yet.
+    mutable LaunchCfg rule[3];
     bool defined() const { return !L.boxes.empty(); }
 };
 
@@ -161,18 +176,6 @@ struct RegridState {
     std::vector<char> no_local, do_global;
     std::vector<double> min_distance, latest;
     long long attempts = 0, global_wanted = 0;
-};
-
-/** Launch shape of the stage kernels.  A field of -1 (tz: 0) is not set:
- *  the level's tuned value, else the default, applies. */
-struct LaunchCfg {
-    int variant = -1;     // tile shape index into kVariants
-    int tz = 0;           // z-chunk length of a tile (0: automatic)
-    int xcd_split = -1;   // each XCD walks one contiguous range of tiles
-    int persistent = -1;  // grid = resident capacity (1) or one tile per workgroup (0)
-    int zc_minor = -1;    // tile order: z-chunk outermost (0) or innermost (1)
-    int fused = -1;       // SSPRK3 stages one and two in one launch (0/1)
-    int fused_variant = -1;  // tile shape of that launch
 };
 
 /** A captured level step (swap excluded): the stage launches and ghost
@@ -319,6 +322,9 @@ class Runtime {
     void bump_epoch() { ++epoch_; }
     /** Launch shape used for level lev (overrides, tuned values, defaults). */
     LaunchCfg resolved_launch(int lev) const;
+    /** Launch shape by the level's box sizes alone (nothing timed); fused: 0
+     *  or 1 fixes whether the first two stages run in one launch. */
+    LaunchCfg rule_launch(const LevelState &ls, int fused) const;
     /** Fused SSPRK3 stages one and two possible at this level (every box
      *  periodic on itself, kernel built for the precision and radius). */
     bool fused_possible(const LevelState &ls) const;
