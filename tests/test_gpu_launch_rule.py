@@ -1,0 +1,59 @@
+"""Launch shapes of levels nobody tuned (a rule on box sizes, precision and
+field count picks the tile, the chunk length and whether the first two stages
+run fused): the same cells bit for bit as the 64 x 8 tile on 16-plane chunks
+with separate stages, on sizes at the edges of tiles and chunks."""
+import numpy as np
+import pytest
+
+import sledgehamr_amd as shm
+from cases import complex_scalar, ensemble_inputs, real_scalar
+
+pytestmark = pytest.mark.gpu
+
+ALLP = [shm.PREC_FP64, shm.PREC_FP32C, shm.PREC_FP32C16, shm.PREC_FP32CS]
+ANY = {"shm.allow_any_grid_size": 1}
+
+
+def _same_as_fixed(project, inp, prec, boxes=None, steps=3):
+    out = []
+    for fixed in (True, False):
+        sim = shm.Simulation(project, inp, precision=prec)
+        if boxes is not None:
+            sim.set_boxes(0, boxes)
+        if fixed:
+            sim.set_launch(variant=1, tile_z=16, fused=0)
+        rng = np.random.default_rng(5)
+        nc = sim.info["ncomp"]
+        for c in range(nc):
+            sim.upload(0, c, 0.3 * rng.standard_normal(sim.ncells(0)) + (c == 0))
+        sim.advance(0, steps)
+        out.append([sim.download(0, c) for c in range(nc)])
+        launch = sim.get_launch(0)
+        sim.close()
+    for c, (a, b) in enumerate(zip(*out)):
+        assert np.isfinite(a).all() and np.array_equal(a, b), c
+    return launch
+
+
+@pytest.mark.parametrize("N", [8, 30, 64, 66, 98, 130])
+@pytest.mark.parametrize("prec", ALLP)
+def test_complex_ssprk3(N, prec):
+    lc = _same_as_fixed("ComplexScalar", complex_scalar(N=N, **ANY), prec)
+    assert lc["fused"] == (1 if N >= 64 and prec != shm.PREC_FP32CS else 0)
+
+
+@pytest.mark.parametrize("order,integrator", [(1, 21), (2, 22), (3, 21), (2, 11)])
+@pytest.mark.parametrize("N", [14, 64, 100])
+@pytest.mark.parametrize("prec", [shm.PREC_FP64, shm.PREC_FP32C16])
+def test_real_scalar(N, order, integrator, prec):
+    _same_as_fixed("RealScalar", real_scalar(N=N, order=order, integrator=integrator, **ANY),
+                   prec)
+
+
+@pytest.mark.parametrize("prec", [shm.PREC_FP64, shm.PREC_FP32C16, shm.PREC_FP32CS])
+@pytest.mark.parametrize("edges", [[(17, 33, 9)], [(17, 33, 9), (64, 8, 70), (5, 65, 31)],
+                                   [(40, 40, 40)] * 30])
+def test_ragged_ensembles(edges, prec):
+    boxes = [[0, 0, 0, a - 1, b - 1, c - 1] for a, b, c in edges]
+    inp = ensemble_inputs([[0, 0, 0, 127, 127, 127]], integrator=21, order=2)
+    _same_as_fixed("RealScalar", inp, prec, boxes)
