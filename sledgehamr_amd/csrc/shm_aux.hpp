@@ -1167,12 +1167,14 @@ __global__ void __launch_bounds__(256) regrid_select_kernel(const RegridArgs a) 
 // ---------------------------------------------------------------------------
 
 /** TO_STATE: dense -> state (leading word and remainder as the stage kernels
- *  store them); else state -> dense (leading word plus remainder). */
+ *  store them); else state -> dense (leading word plus remainder).  Downloads
+ *  pass pinned host memory as `dense`, so the values cross the bus as they
+ *  are formed: no dense device copy of the component, no second pass. */
 template <Prec P, bool TO_STATE>
 __global__ void __launch_bounds__(256) valid_io_kernel(const ValidIoArgs a) {
     using T = PrecTraits<P>;
     const long long stride = (long long)gridDim.x * blockDim.x;
-    for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < a.total;
+    for (long long t = a.first + (long long)blockIdx.x * blockDim.x + threadIdx.x; t < a.total;
          t += stride) {
         int lo = 0, hi = a.nbox - 1;
         while (lo < hi) {
@@ -1183,14 +1185,16 @@ __global__ void __launch_bounds__(256) valid_io_kernel(const ValidIoArgs a) {
                 hi = mid - 1;
         }
         const BoxDesc &b = a.boxes[lo];
-        const long long r = t - a.vprefix[lo];
-        const long long row = r / b.n[0];
-        const long long e = a.comp_off + b.base + (r - row * b.n[0]) +
-                            (row % b.n[1]) * b.jstride + (row / b.n[1]) * b.kstride;
+        // A box holds fewer than 2^32 cells (its brick offsets are 32-bit).
+        const unsigned r = (unsigned)(t - a.vprefix[lo]);
+        const unsigned row = r / (unsigned)b.n[0], z = row / (unsigned)b.n[1];
+        const long long e = a.comp_off + b.base + (r - row * (unsigned)b.n[0]) +
+                            (long long)(row - z * (unsigned)b.n[1]) * b.jstride +
+                            (long long)z * b.kstride;
         if constexpr (TO_STATE)
-            store_state_at<T>(a.hi, a.lo, e, a.dense[t]);
+            store_state_at<T>(a.hi, a.lo, e, a.dense[t - a.first]);
         else
-            a.dense[t] = load_state_at<T>(a.hi, a.lo, e);
+            a.dense[t - a.first] = load_state_at<T>(a.hi, a.lo, e);
     }
 }
 

@@ -6,6 +6,7 @@
 #include <sledgehamr.h>
 
 #include <array>
+#include <functional>
 #include <cfloat>
 #include <map>
 #include <set>
@@ -420,6 +421,15 @@ class Runtime {
     /** Valid cells of component comp_id of state `which`: from the host
      *  array (to_state) or into it, in one kernel and one copy. */
     void valid_io(LevelState &ls, int comp_id, int which, double *host, bool to_state);
+    /** Moves nbytes produced on the device into pageable host memory through
+     *  a ring of pinned slots: produce(offset, bytes, slot, the slot as the
+     *  device addresses it) enqueues on the stream what writes those bytes
+     *  into a slot (a kernel or a copy), and threads of this call copy
+     *  finished slots on while the next ones are produced.  Returns when dst
+     *  is complete. */
+    void to_host(void *dst, size_t nbytes,
+                 const std::function<void(size_t, size_t, void *, void *)> &produce);
+    int device_ = 0;
     /** The coarsened copy of level lev (>= 1) on level lev-1, built once
      *  per epoch with its copy plans. */
     LevelState &coarse_mirror(int lev);
