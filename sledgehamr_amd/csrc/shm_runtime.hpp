@@ -82,9 +82,16 @@ struct Layout {
     int g = 0;          // ghost width
     bool periodic = true;
     bool independent = false;  // every box is its own periodic domain
-    std::vector<Box3> boxes;
+    std::vector<Box3> boxes;   // the level's boxes: data order, tags, copy plans
     std::vector<BoxDesc> hbox;
     DevMem dbox;
+    // What is stored and stepped: the boxes themselves, or, where they tile
+    // the whole periodic domain, one brick of the domain that every box is a
+    // window of.  Ghost cells exist around these only.
+    bool merged = false;
+    std::vector<Box3> sboxes;
+    std::vector<BoxDesc> hsbox;
+    DevMem dsbox;
     long long cstride = 0;  // elements per component plane
     std::vector<long long> vprefix;  // valid cells per box (prefix, nbox+1)
     DevMem dvprefix;
@@ -98,8 +105,10 @@ struct Layout {
     long long halo_full_total = 0;
     std::map<std::tuple<int, int, int, int>, std::pair<std::shared_ptr<DevMem>, int>> tiles;
 
+    /** may_merge: boxes that tile the domain may be stored as one brick (not
+     *  for levels whose ghost cells a coarser level fills box by box). */
     void build(const std::vector<Box3> &b, int ghost, int domain_n,
-               bool is_periodic, bool is_independent = false);
+               bool is_periodic, bool is_independent = false, bool may_merge = false);
     const TileDesc *get_tiles(int ty, int tz, int zc_minor, int *ntiles, int tx = 64);
     long long nvalid() const { return vprefix.empty() ? 0 : vprefix.back(); }
 };
