@@ -363,10 +363,28 @@ struct Walk3 {
     }
 };
 
+/** A workgroup fills the ghost cells of one tile of coarse parents, one
+ *  component after the other: the tile's coarse brick (its parents grown by
+ *  the stencil reach) goes to LDS as time-weighted FP64 values, then one
+ *  thread per parent forms its interpolation coefficients once and writes
+ *  its children.
+ *
+ *  What bounds it: waiting.  A shell tile is small (at most 256 parents) and
+ *  its work a chain of load, barrier, LDS reads, stores; the values written
+ *  (1.05 GB for 22 M ghost cells of a level of 2000 boxes) take 0.2 ms at the
+ *  memory rate.  So the chain is kept short: the coarse cell of each of a
+ *  thread's brick points is looked up once, not per component; the next
+ *  component's coarse words are loaded while a component is interpolated;
+ *  coefficients are formed per parent, not per child (24 children values of
+ *  19 LDS reads each were 456 reads, now 57); the two x children of a parent
+ *  leave in one store; thin slabs have tiles that are long in their plane
+ *  (a 1 x 8 x 4 tile kept 32 of 256 threads busy).  A coarse step of the
+ *  256^3 base with two levels of 2000 boxes: 43.0 to 33.6 ms. */
 template <Prec P, int MODE, int INTERP>
 __global__ void __launch_bounds__(256) cf_fill_kernel(const CfArgs a) {
     using T = PrecTraits<P>;
     using S = typename T::S;
+    using LO = typename T::L;
     // Stage states are composed in the tile type V from u0's tile value (the
     // leading word for FP32 tiles, hi + lo for FP64 tiles) and coefficients
     // in V: the ghost values below compose to the interpolated state the
@@ -399,7 +417,7 @@ __global__ void __launch_bounds__(256) cf_fill_kernel(const CfArgs a) {
     // brick each).
     constexpr int NTIME = MODE == kCfSsprk ? 3 : 1;
     double twO[NTIME], twN[NTIME];
-    bool tuO[NTIME], tuN[NTIME];
+    bool tuO[NTIME], tuN[NTIME], any_new = false, any_old = false;
 #pragma unroll
     for (int ti = 0; ti < NTIME; ++ti) {
         const double *rc = ti == 0 ? a.rec : a.rec3[ti - 1];
@@ -407,37 +425,77 @@ __global__ void __launch_bounds__(256) cf_fill_kernel(const CfArgs a) {
         twN[ti] = rc[1];
         tuO[ti] = rc[2] != 0.;
         tuN[ti] = rc[3] != 0.;
+        any_new = any_new || tuN[ti];
+        any_old = any_old || tuO[ti];
     }
-    const double wo = a.rec[0], wn = a.rec[1];
-    const bool use_old = a.rec[2] != 0., use_new = a.rec[3] != 0.;
     const int ns = a.rec[4] != 0. ? 1 : 0;
     const void *cnew = a.cs[ns], *cnewlo = a.cslo[ns];
     const void *cold = a.cs[ns ^ 1], *coldlo = a.cslo[ns ^ 1];
-    auto cval = [&](int comp, long long ce) -> double {
-        const long long e = (long long)comp * a.ccstride + ce;
-        double v = 0.;
-        if (use_new) v = load_state_at<T>(cnew, cnewlo, e);
-        if (use_old) {
-            const double vo = load_state_at<T>(cold, coldlo, e);
-            v = use_new ? wo * vo + wn * v : vo;
+
+    // This thread's brick points (threadIdx.x, + 256, ...; a brick holds at
+    // most kCfBrick) and their coarse elements in a component plane: the
+    // periodic image of each coarse cell in the candidate boxes of the fine
+    // box (every one is held: nesting is checked when the plan is built).
+    constexpr int CPT = kCfBrick / 256;
+    long long ce[CPT];
+    {
+        int hint = 0;
+        Walk3 w(threadIdx.x, 256, bxn, byn);
+#pragma unroll
+        for (int c = 0; c < CPT; ++c) {
+            ce[c] = -1;
+            if ((int)threadIdx.x + 256 * c < nb) {
+                const int ci = cf_wrap(tl.plo[0] - R + w.x, a.Nc);
+                const int cj = cf_wrap(tl.plo[1] - R + w.y, a.Nc);
+                const int ck = cf_wrap(tl.plo[2] - R + w.z, a.Nc);
+                for (int k = 0; k < ncand && ce[c] < 0; ++k) {
+                    const int qq = hint + k < ncand ? hint + k : hint + k - ncand;
+                    const BoxDesc &cb = a.cboxes[a.cand[cs0 + qq]];
+                    if (ci >= cb.lo[0] && ci < cb.lo[0] + cb.n[0] && cj >= cb.lo[1] &&
+                        cj < cb.lo[1] + cb.n[1] && ck >= cb.lo[2] && ck < cb.lo[2] + cb.n[2]) {
+                        ce[c] = cb.base + (ci - cb.lo[0]) +
+                                (long long)(cj - cb.lo[1]) * cb.jstride +
+                                (long long)(ck - cb.lo[2]) * cb.kstride;
+                        hint = qq;
+                    }
+                }
+            }
+            w.next();
         }
-        return v;
+    }
+    // Raw coarse words of a component at those points.
+    S hn[CPT], ho[CPT];
+    LO ln[CPT], lo_[CPT];
+    auto fetch = [&](int n) {
+        const long long cp = (long long)a.comp[n] * a.ccstride;
+#pragma unroll
+        for (int c = 0; c < CPT; ++c) {
+            hn[c] = ho[c] = S();
+            ln[c] = lo_[c] = LO();
+            if (ce[c] < 0) continue;
+            const long long e = cp + ce[c];
+            if (any_new) {
+                hn[c] = ld<S>(cnew, e, 0u);
+                if constexpr (T::comp) ln[c] = ld_nt<LO>(cnewlo, e, 0u);
+            }
+            if (any_old) {
+                ho[c] = ld<S>(cold, e, 0u);
+                if constexpr (T::comp) lo_[c] = ld_nt<LO>(coldlo, e, 0u);
+            }
+        }
+    };
+    auto whole = [](S h, LO l) -> double {  // as load_state reads the pair
+        if constexpr (!T::comp)
+            return (double)h + 0.;
+        else if constexpr (std::is_same_v<LO, float>)
+            return (double)h + (double)l;
+        else
+            return (double)h + (double)bf16_to_f32(l);
     };
     // What the ghost cell at fine element fe receives for component slot n.
     auto put = [&](int n, long long fe, double v) {
         const int comp = a.comp[n];
-        if constexpr (MODE == kCfState) {
-            const long long e = (long long)comp * a.fcstride + fe;
-            // Without a remainder array (dstlo null) only the leading word.
-            if constexpr (T::comp) {
-                if (a.dstlo)
-                    store_state_at<T>(a.dst, a.dstlo, e, v);
-                else
-                    st<float>(a.dst, e, 0u, (float)v);
-            } else {
-                store_state_at<T>(a.dst, a.dstlo, e, v);
-            }
-        } else if constexpr (MODE == kCfK) {
+        if constexpr (MODE == kCfK) {
             const long long e = (long long)comp * a.fcstride + fe;
             const double u0 = u0_at(e);
             st<S>(a.dst, e, 0u, (S)((v - u0) / (double)(V)a.c0));
@@ -450,46 +508,55 @@ __global__ void __launch_bounds__(256) cf_fill_kernel(const CfArgs a) {
             st<S>(a.dst, pe, 0u, (S)((v - yv) / (double)(V)a.cf[a.m]));
         }
     };
+    // The two x children of a parent at element e (lower child) in one store;
+    // both: they are in the slab and e is even, else each by itself.
+    auto put2 = [](auto *arr, long long e, auto v0, auto v1, bool in0, bool in1, bool both) {
+        using X = decltype(v0);
+        typedef X X2 __attribute__((ext_vector_type(2)));
+        X *p = static_cast<X *>(static_cast<void *>(arr)) + e;
+        if (both) {
+            *reinterpret_cast<X2 *>(p) = X2{v0, v1};
+        } else {
+            if (in0) p[0] = v0;
+            if (in1) p[1] = v1;
+        }
+    };
+    auto put2_state = [&](long long e, double v0, double v1, bool in0, bool in1, bool both) {
+        if constexpr (T::comp) {
+            const float h0 = (float)v0, h1 = (float)v1;
+            put2((char *)a.dst, e, h0, h1, in0, in1, both);
+            if (a.dstlo) {  // null: only the leading words
+                const float r0 = (float)(v0 - (double)h0), r1 = (float)(v1 - (double)h1);
+                if constexpr (std::is_same_v<LO, float>)
+                    put2((char *)a.dstlo, e, r0, r1, in0, in1, both);
+                else
+                    put2((char *)a.dstlo, e, f32_to_bf16_rne(r0), f32_to_bf16_rne(r1), in0, in1,
+                         both);
+            }
+        } else {
+            put2((char *)a.dst, e, (S)v0, (S)v1, in0, in1, both);
+        }
+    };
+
+    fetch(0);
     for (int n = 0; n < a.ncomp; ++n) {
         const int comp = a.comp[n];
         __syncthreads();  // the previous component's brick has been read
-        // Brick cells, coalesced along x: the periodic image of each coarse
-        // cell in the candidate boxes of the fine box (every one is held:
-        // nesting is checked when the plan is built).
-        int hint = 0;
-        Walk3 w(threadIdx.x, blockDim.x, bxn, byn);
-        for (int q = threadIdx.x; q < nb; q += blockDim.x, w.next()) {
-            const int ci = cf_wrap(tl.plo[0] - R + w.x, a.Nc);
-            const int cj = cf_wrap(tl.plo[1] - R + w.y, a.Nc);
-            const int ck = cf_wrap(tl.plo[2] - R + w.z, a.Nc);
-            long long e = -1;
-            for (int k = 0; k < ncand && e < 0; ++k) {
-                const int qq = hint + k < ncand ? hint + k : hint + k - ncand;
-                const BoxDesc &cb = a.cboxes[a.cand[cs0 + qq]];
-                if (ci >= cb.lo[0] && ci < cb.lo[0] + cb.n[0] && cj >= cb.lo[1] &&
-                    cj < cb.lo[1] + cb.n[1] && ck >= cb.lo[2] && ck < cb.lo[2] + cb.n[2]) {
-                    e = cb.base + (ci - cb.lo[0]) + (long long)(cj - cb.lo[1]) * cb.jstride +
-                        (long long)(ck - cb.lo[2]) * cb.kstride;
-                    hint = qq;
-                }
-            }
-            if constexpr (MODE == kCfSsprk) {
-                // Both coarse states once, weighted per time as cval does.
-                double vn = 0., vo = 0.;
-                const long long ce = (long long)comp * a.ccstride + (e >= 0 ? e : 0);
-                if (tuN[0] || tuN[1] || tuN[2]) vn = load_state_at<T>(cnew, cnewlo, ce);
-                if (tuO[0] || tuO[1] || tuO[2]) vo = load_state_at<T>(cold, coldlo, ce);
 #pragma unroll
-                for (int ti = 0; ti < NTIME; ++ti) {
-                    double v = 0.;
-                    if (tuN[ti]) v = vn;
-                    if (tuO[ti]) v = tuN[ti] ? twO[ti] * vo + twN[ti] * v : vo;
-                    brick[ti * nb + q] = e >= 0 ? v : __builtin_nan("");
-                }
-            } else {
-                brick[q] = e >= 0 ? cval(comp, e) : __builtin_nan("");
+        for (int c = 0; c < CPT; ++c) {
+            const int q = threadIdx.x + 256 * c;
+            if (q >= nb) continue;
+            const double vn = any_new ? whole(hn[c], ln[c]) : 0.;
+            const double vo = any_old ? whole(ho[c], lo_[c]) : 0.;
+#pragma unroll
+            for (int ti = 0; ti < NTIME; ++ti) {
+                double v = 0.;
+                if (tuN[ti]) v = vn;
+                if (tuO[ti]) v = tuN[ti] ? twO[ti] * vo + twN[ti] * v : vo;
+                brick[ti * nb + q] = ce[c] >= 0 ? v : __builtin_nan("");
             }
         }
+        if (n + 1 < a.ncomp) fetch(n + 1);
         __syncthreads();
         Walk3 pw(threadIdx.x, blockDim.x, tl.pn[0], tl.pn[1]);
         for (int p = threadIdx.x; p < np; p += blockDim.x, pw.next()) {
@@ -503,184 +570,147 @@ __global__ void __launch_bounds__(256) cf_fill_kernel(const CfArgs a) {
                 c1[d] = min(1, sg.flo[d] + sg.fn[d] - 1 - 2 * pc[d]);
             }
             const int b0 = (px + R) + bxn * ((py + R) + byn * (pz + R));
-            auto C = [&](int di, int dj, int dk) -> double {
-                return brick[b0 + di + bxn * (dj + byn * dk)];
-            };
-            auto fine_elem = [&](int cx, int cy, int cz) -> long long {
-                return db.base + (2 * pc[0] + cx - db.lo[0]) +
-                       (long long)(2 * pc[1] + cy - db.lo[1]) * db.jstride +
-                       (long long)(2 * pc[2] + cz - db.lo[2]) * db.kstride;
-            };
-            if constexpr (MODE == kCfSsprk) {
-                // The interpolated value of child (x, y, z) from brick bb,
-                // by the same expressions as the per-parent forms below.
-                auto value = [&](const double *bb, int x, int y, int z) -> double {
-                    auto Cb = [&](int di, int dj, int dk) -> double {
-                        return bb[b0 + di + bxn * (dj + byn * dk)];
+            // Fine element of child (0, 0, 0) in a component plane.
+            const long long f0 = db.base + (2 * pc[0] - db.lo[0]) +
+                                 (long long)(2 * pc[1] - db.lo[1]) * db.jstride +
+                                 (long long)(2 * pc[2] - db.lo[2]) * db.kstride;
+            const bool in0 = c0[0] == 0, in1 = c1[0] == 1;
+            // (Row and plane pitches are even.)
+            const bool both = in0 && in1 && (f0 & 1) == 0;
+            // Values of the eight children from brick bb.
+            auto children = [&](const double *bb, double (&v)[2][2][2]) {
+                auto C = [&](int di, int dj, int dk) -> double {
+                    return bb[b0 + di + bxn * (dj + byn * dk)];
+                };
+                if constexpr (INTERP == 4) {
+                    // Tensor product of the conservative quartic child
+                    // weights; an upper child (odd fine index) takes WU, a
+                    // lower one its mirror.
+                    // WU = (3, -22, 128, 22, -3) / 128 as selects (no
+                    // indexed array, which would live in scratch memory).
+                    auto wu = [](int q) -> double {
+                        return q == 0 ? 3. / 128. : q == 1 ? -22. / 128. : q == 2 ? 1.
+                                                  : q == 3 ? 22. / 128. : -3. / 128.;
                     };
-                    if constexpr (INTERP == 4) {
-                        auto wu = [](int q) -> double {
-                            return q == 0 ? 3. / 128. : q == 1 ? -22. / 128. : q == 2 ? 1.
-                                                      : q == 3 ? 22. / 128. : -3. / 128.;
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) v[q >> 2][(q >> 1) & 1][q & 1] = 0.;
+#pragma unroll 1
+                    for (int cz = 0; cz < 5; ++cz)
+#pragma unroll 1
+                        for (int by = 0; by < 5; ++by)
+#pragma unroll
+                            for (int ax = 0; ax < 5; ++ax) {
+                                const double cv = C(ax - 2, by - 2, cz - 2);
+                                const double wz[2] = {wu(4 - cz), wu(cz)};
+                                const double wy[2] = {wu(4 - by), wu(by)};
+                                const double wx[2] = {wu(4 - ax), wu(ax)};
+#pragma unroll
+                                for (int z = 0; z < 2; ++z)
+#pragma unroll
+                                    for (int y = 0; y < 2; ++y)
+#pragma unroll
+                                        for (int x = 0; x < 2; ++x)
+                                            v[z][y][x] += wz[z] * wy[y] * wx[x] * cv;
+                            }
+                } else {
+                    double c[NPT];
+#pragma unroll
+                    for (int q = 0; q < NPT; ++q) c[q] = C(PO[q][0], PO[q][1], PO[q][2]);
+                    // Slopes of the parent, shared by its children at x, y, z =
+                    // +-1/4 coarse cells.
+                    double sx = 0., sy = 0., sz = 0., sxx = 0., syy = 0., szz = 0., sxy = 0.,
+                           sxz = 0., syz = 0.;
+                    if constexpr (INTERP == 2) {
+                        sx = 0.5 * (c[2] - c[1]);
+                        sy = 0.5 * (c[4] - c[3]);
+                        sz = 0.5 * (c[6] - c[5]);
+                        sxx = 0.5 * (c[2] - 2. * c[0] + c[1]);
+                        syy = 0.5 * (c[4] - 2. * c[0] + c[3]);
+                        szz = 0.5 * (c[6] - 2. * c[0] + c[5]);
+                        sxy = 0.25 * (c[7] - c[8] - c[9] + c[10]);
+                        sxz = 0.25 * (c[11] - c[12] - c[13] + c[14]);
+                        syz = 0.25 * (c[15] - c[16] - c[17] + c[18]);
+                    } else if constexpr (INTERP == 1) {
+                        // Monotonized-central slopes per direction.
+                        auto mc = [](double cm, double c0v, double cp) {
+                            const double sl = c0v - cm, sr = cp - c0v;
+                            const double sc = 0.5 * (sl + sr);
+                            if (!(sl * sr > 0.)) return 0.;
+                            const double m = fmin(fabs(sc), fmin(2. * fabs(sl), 2. * fabs(sr)));
+                            return sc > 0. ? m : -m;
                         };
-                        double acc = 0.;
-#pragma unroll 1
-                        for (int cz = 0; cz < 5; ++cz)
-#pragma unroll 1
-                            for (int by = 0; by < 5; ++by)
+                        sx = mc(c[1], c[0], c[2]);
+                        sy = mc(c[3], c[0], c[4]);
+                        sz = mc(c[5], c[0], c[6]);
+                    }
 #pragma unroll
-                                for (int ax = 0; ax < 5; ++ax) {
-                                    const double wz = z ? wu(cz) : wu(4 - cz);
-                                    const double wy = y ? wu(by) : wu(4 - by);
-                                    const double wx = x ? wu(ax) : wu(4 - ax);
-                                    acc += wz * wy * wx * Cb(ax - 2, by - 2, cz - 2);
-                                }
-                        return acc;
-                    } else {
-                        double c[NPT];
-#pragma unroll
-                        for (int q = 0; q < NPT; ++q) c[q] = Cb(PO[q][0], PO[q][1], PO[q][2]);
+                    for (int q = 0; q < 8; ++q) {
+                        const int x = q & 1, y = (q >> 1) & 1, z = q >> 2;
                         const double xo = x ? 0.25 : -0.25, yo = y ? 0.25 : -0.25,
                                      zo = z ? 0.25 : -0.25;
-                        if constexpr (INTERP == 2) {
-                            const double sx = 0.5 * (c[2] - c[1]), sy = 0.5 * (c[4] - c[3]),
-                                         sz = 0.5 * (c[6] - c[5]);
-                            const double sxx = 0.5 * (c[2] - 2. * c[0] + c[1]);
-                            const double syy = 0.5 * (c[4] - 2. * c[0] + c[3]);
-                            const double szz = 0.5 * (c[6] - 2. * c[0] + c[5]);
-                            const double sxy = 0.25 * (c[7] - c[8] - c[9] + c[10]);
-                            const double sxz = 0.25 * (c[11] - c[12] - c[13] + c[14]);
-                            const double syz = 0.25 * (c[15] - c[16] - c[17] + c[18]);
-                            return c[0] + xo * sx + yo * sy + zo * sz + xo * xo * sxx +
-                                   yo * yo * syy + zo * zo * szz + xo * yo * sxy +
-                                   xo * zo * sxz + yo * zo * syz;
-                        } else if constexpr (INTERP == 1) {
-                            auto mc = [](double cm, double c0v, double cp) {
-                                const double sl = c0v - cm, sr = cp - c0v;
-                                const double sc = 0.5 * (sl + sr);
-                                if (!(sl * sr > 0.)) return 0.;
-                                const double m =
-                                    fmin(fabs(sc), fmin(2. * fabs(sl), 2. * fabs(sr)));
-                                return sc > 0. ? m : -m;
-                            };
-                            return c[0] + xo * mc(c[1], c[0], c[2]) +
-                                   yo * mc(c[3], c[0], c[4]) + zo * mc(c[5], c[0], c[6]);
-                        } else {
-                            return c[0];
-                        }
+                        if constexpr (INTERP == 2)
+                            v[z][y][x] = c[0] + xo * sx + yo * sy + zo * sz + xo * xo * sxx +
+                                         yo * yo * syy + zo * zo * szz + xo * yo * sxy +
+                                         xo * zo * sxz + yo * zo * syz;
+                        else if constexpr (INTERP == 1)
+                            v[z][y][x] = c[0] + xo * sx + yo * sy + zo * sz;
+                        else
+                            v[z][y][x] = c[0];
                     }
-                };
-                // u0 at t0 (its leading word; with FP64 tiles of stored
-                // pairs hi and lo), then k1 and k2 such that u0 + dt k1 and
-                // u0 + dt/4 k2 are the states at t0 + dt and t0 + dt/2, as
-                // the separate state and k fills write them.
-                for (int z = c0[2]; z <= c1[2]; ++z)
-                    for (int y = c0[1]; y <= c1[1]; ++y)
-                        for (int x = c0[0]; x <= c1[0]; ++x) {
-                            const long long e = (long long)comp * a.fcstride + fine_elem(x, y, z);
-                            const double u0v = value(brick, x, y, z);
-                            double u0t;  // u0's tile value as the stage kernels read it
-                            if constexpr (T::comp && T::exact) {
-                                store_state_at<T>(a.dst, a.dstlo, e, u0v);
-                                u0t = pair_value<T>(u0v);
+                }
+            };
+            double v[2][2][2];
+            if constexpr (MODE == kCfSsprk) {
+                // u0 at t0 (its leading word; with FP64 tiles of stored pairs
+                // hi and lo), then k1 and k2 such that u0 + dt k1 and
+                // u0 + dt/4 k2 are the states at t0 + dt and t0 + dt/2.
+                const long long e0 = (long long)comp * a.fcstride + f0;
+                double u0t[2][2][2];  // u0's tile values as the stage kernels read them
+                children(brick, u0t);
+#pragma unroll
+                for (int ti = 0; ti < 3; ++ti) {
+                    if (ti > 0) children(brick + ti * nb, v);
+#pragma unroll
+                    for (int z = 0; z < 2; ++z)
+#pragma unroll
+                        for (int y = 0; y < 2; ++y) {
+                            if (z < c0[2] || z > c1[2] || y < c0[1] || y > c1[1]) continue;
+                            const long long e = e0 + (long long)y * db.jstride +
+                                                (long long)z * db.kstride;
+                            double *u = u0t[z][y];
+                            if (ti > 0) {
+                                const double cf = (double)(V)a.cf[ti - 1];
+                                put2((char *)a.kd[ti - 1], e, (S)((v[z][y][0] - u[0]) / cf),
+                                     (S)((v[z][y][1] - u[1]) / cf), in0, in1, both);
+                            } else if constexpr (T::comp && T::exact) {
+                                put2_state(e, u[0], u[1], in0, in1, both);
+                                u[0] = pair_value<T>(u[0]);
+                                u[1] = pair_value<T>(u[1]);
                             } else {
-                                const S u0s = (S)u0v;
-                                st<S>(a.dst, e, 0u, u0s);
-                                u0t = (double)u0s;
+                                const S h0 = (S)u[0], h1 = (S)u[1];
+                                put2((char *)a.dst, e, h0, h1, in0, in1, both);
+                                u[0] = (double)h0;
+                                u[1] = (double)h1;
                             }
-                            st<S>(a.kd[0], e, 0u,
-                                  (S)((value(brick + nb, x, y, z) - u0t) /
-                                      (double)(V)a.cf[0]));
-                            st<S>(a.kd[1], e, 0u,
-                                  (S)((value(brick + 2 * nb, x, y, z) - u0t) /
-                                      (double)(V)a.cf[1]));
                         }
-            } else if constexpr (INTERP == 4) {
-                // Tensor product of the conservative quartic child weights;
-                // an upper child (odd fine index) takes WU, a lower one its
-                // mirror.
-                // WU = (3, -22, 128, 22, -3) / 128 as selects (no indexed
-                // array, which would live in scratch memory).
-                auto wu = [](int q) -> double {
-                    return q == 0 ? 3. / 128. : q == 1 ? -22. / 128. : q == 2 ? 1.
-                                              : q == 3 ? 22. / 128. : -3. / 128.;
-                };
-                double acc[2][2][2] = {{{0., 0.}, {0., 0.}}, {{0., 0.}, {0., 0.}}};
-#pragma unroll 1
-                for (int cz = 0; cz < 5; ++cz)
-#pragma unroll 1
-                    for (int by = 0; by < 5; ++by)
-#pragma unroll
-                        for (int ax = 0; ax < 5; ++ax) {
-                            const double v = C(ax - 2, by - 2, cz - 2);
-                            const double wz[2] = {wu(4 - cz), wu(cz)};
-                            const double wy[2] = {wu(4 - by), wu(by)};
-                            const double wx[2] = {wu(4 - ax), wu(ax)};
-#pragma unroll
-                            for (int z = 0; z < 2; ++z)
-#pragma unroll
-                                for (int y = 0; y < 2; ++y)
-#pragma unroll
-                                    for (int x = 0; x < 2; ++x)
-                                        acc[z][y][x] += wz[z] * wy[y] * wx[x] * v;
-                        }
-                // Compile-time child indices keep acc in registers.
+                }
+            } else {
+                children(brick, v);
 #pragma unroll
                 for (int z = 0; z < 2; ++z)
 #pragma unroll
-                    for (int y = 0; y < 2; ++y)
-#pragma unroll
-                        for (int x = 0; x < 2; ++x)
-                            if (z >= c0[2] && z <= c1[2] && y >= c0[1] && y <= c1[1] &&
-                                x >= c0[0] && x <= c1[0])
-                                put(n, fine_elem(x, y, z), acc[z][y][x]);
-            } else {
-                double c[NPT];
-#pragma unroll
-                for (int q = 0; q < NPT; ++q) c[q] = C(PO[q][0], PO[q][1], PO[q][2]);
-                // Slopes of the parent, shared by its children at x, y, z =
-                // +-1/4 coarse cells.
-                double sx = 0., sy = 0., sz = 0., sxx = 0., syy = 0., szz = 0., sxy = 0.,
-                       sxz = 0., syz = 0.;
-                if constexpr (INTERP == 2) {
-                    sx = 0.5 * (c[2] - c[1]);
-                    sy = 0.5 * (c[4] - c[3]);
-                    sz = 0.5 * (c[6] - c[5]);
-                    sxx = 0.5 * (c[2] - 2. * c[0] + c[1]);
-                    syy = 0.5 * (c[4] - 2. * c[0] + c[3]);
-                    szz = 0.5 * (c[6] - 2. * c[0] + c[5]);
-                    sxy = 0.25 * (c[7] - c[8] - c[9] + c[10]);
-                    sxz = 0.25 * (c[11] - c[12] - c[13] + c[14]);
-                    syz = 0.25 * (c[15] - c[16] - c[17] + c[18]);
-                } else if constexpr (INTERP == 1) {
-                    // Monotonized-central slopes per direction.
-                    auto mc = [](double cm, double c0v, double cp) {
-                        const double sl = c0v - cm, sr = cp - c0v;
-                        const double sc = 0.5 * (sl + sr);
-                        if (!(sl * sr > 0.)) return 0.;
-                        const double m = fmin(fabs(sc), fmin(2. * fabs(sl), 2. * fabs(sr)));
-                        return sc > 0. ? m : -m;
-                    };
-                    sx = mc(c[1], c[0], c[2]);
-                    sy = mc(c[3], c[0], c[4]);
-                    sz = mc(c[5], c[0], c[6]);
-                }
-                for (int z = c0[2]; z <= c1[2]; ++z)
-                    for (int y = c0[1]; y <= c1[1]; ++y)
-                        for (int x = c0[0]; x <= c1[0]; ++x) {
-                            const double xo = x ? 0.25 : -0.25, yo = y ? 0.25 : -0.25,
-                                         zo = z ? 0.25 : -0.25;
-                            double v;
-                            if constexpr (INTERP == 2)
-                                v = c[0] + xo * sx + yo * sy + zo * sz + xo * xo * sxx +
-                                    yo * yo * syy + zo * zo * szz + xo * yo * sxy +
-                                    xo * zo * sxz + yo * zo * syz;
-                            else if constexpr (INTERP == 1)
-                                v = c[0] + xo * sx + yo * sy + zo * sz;
-                            else
-                                v = c[0];
-                            put(n, fine_elem(x, y, z), v);
+                    for (int y = 0; y < 2; ++y) {
+                        if (z < c0[2] || z > c1[2] || y < c0[1] || y > c1[1]) continue;
+                        const long long e = f0 + (long long)y * db.jstride +
+                                            (long long)z * db.kstride;
+                        if constexpr (MODE == kCfState) {
+                            put2_state((long long)comp * a.fcstride + e, v[z][y][0], v[z][y][1],
+                                       in0, in1, both);
+                        } else {
+                            if (in0) put(n, e, v[z][y][0]);
+                            if (in1) put(n, e + 1, v[z][y][1]);
                         }
+                    }
             }
         }
     }

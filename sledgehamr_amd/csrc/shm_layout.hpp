@@ -65,6 +65,9 @@ struct CfPSeg {
     long long start;  // prefix sum of parent cells
 };
 
+/** Most coarse cells in the brick of a tile (parents grown by the reach). */
+constexpr int kCfBrick = 2048;
+
 /** A workgroup's share of a CfPSeg: parents plo .. plo + pn - 1. */
 struct CfTile {
     int seg;

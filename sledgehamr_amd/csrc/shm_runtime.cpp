@@ -1539,14 +1539,20 @@ void Runtime::build_cf(int lev) {
     upload_vec(ls.dcf_full, ls.cf_full);
     upload_vec(ls.dcf_step, ls.cf_step);
     // Workgroup tiles: at most 32 x 8 x 4 parents (16 x 8 x 4 for the
-    // quartic's reach 2), so the coarse brick of a tile, its parents grown
-    // by the reach, takes at most 16 KB of LDS as doubles and several
-    // workgroups share a CU.
+    // quartic's reach 2) of a whole box, and as many as a workgroup has
+    // threads of a shell slab one or two parents thick, long in its plane;
+    // the brick of a tile, its parents grown by the reach, stays within
+    // kCfBrick cells.
     auto tile = [s](const std::vector<CfPSeg> &v, DevMem &d, int &n, int &lds) {
-        const int lim[3] = {s > 1 ? 16 : 32, 8, 4};
         std::vector<CfTile> t;
         lds = 0;
-        for (int q = 0; q < (int)v.size(); ++q)
+        for (int q = 0; q < (int)v.size(); ++q) {
+            const int *pn = v[q].pn;
+            const std::array<int, 3> lim =
+                pn[0] <= 2   ? std::array<int, 3>{2, 16, 8}
+                : pn[1] <= 2 ? std::array<int, 3>{32, 2, s > 1 ? 4 : 8}
+                : pn[2] <= 2 ? std::array<int, 3>{32, s > 1 ? 4 : 8, 2}
+                             : std::array<int, 3>{s > 1 ? 16 : 32, 8, 4};
             for (int z = 0; z < v[q].pn[2]; z += lim[2])
                 for (int y = 0; y < v[q].pn[1]; y += lim[1])
                     for (int x = 0; x < v[q].pn[0]; x += lim[0]) {
@@ -1559,9 +1565,11 @@ void Runtime::build_cf(int lev) {
                             c.pn[a] = std::min(lim[a], v[q].pn[a] - o[a]);
                             cells *= c.pn[a] + 2 * s;
                         }
+                        if (cells > kCfBrick) throw Error(5, "coarse/fine brick too large");
                         lds = std::max(lds, cells);
                         t.push_back(c);
                     }
+        }
         if (t.size() > (size_t)INT_MAX) throw Error(1, "too many coarse/fine tiles");
         n = (int)t.size();
         upload_vec(d, t);
