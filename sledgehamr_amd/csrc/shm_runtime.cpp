@@ -1051,8 +1051,8 @@ LaunchCfg Runtime::resolved_launch(int lev) const {
     LaunchCfg c;
     c.variant = pick(launch.variant, t.variant, r.variant, kDefaultVariant);
     c.tz = launch.tz > 0 ? launch.tz : t.tz > 0 ? t.tz : r.tz;
-    c.xcd_split = pick(launch.xcd_split, t.xcd_split, -1, 1);
-    c.persistent = pick(launch.persistent, t.persistent, -1, 1);
+    c.xcd_split = pick(launch.xcd_split, t.xcd_split, r.xcd_split, 1);
+    c.persistent = pick(launch.persistent, t.persistent, r.persistent, 1);
     c.zc_minor = pick(launch.zc_minor, t.zc_minor, -1, 0);
     c.fused = pick(launch.fused, t.fused, r.fused, 0);
     int dv = -1;
@@ -1076,10 +1076,26 @@ LaunchCfg Runtime::rule_launch(const LevelState &ls, int fused) const {
     c.variant = kDefaultVariant;
     c.fused = 0;
     const auto &boxes = ls.L.sboxes;
-    // GW levels run as component groups and dissipation is built for one
-    // tile shape: the default with its automatic chunk length is within 1 %
-    // of the autotuner's pick there (384^3: 6.74 against 6.69 ms).
-    if (gw_ || ko_ || boxes.empty()) return c;
+    // Dissipation is built for one tile shape.
+    if (ko_ || boxes.empty()) return c;
+    if (gw_) {
+        // GW levels run as component groups, nine launches a step with few
+        // wavefronts resident each: chunks short enough for two tiles per CU
+        // (32^3..64^3: 250 to 83-100 us per RKN4 step on 32 x 8 tiles of 4
+        // planes, 96^3 246 to 186, 128^3 342 to 310, 192^3 995 to 961).  From
+        // 256^3 up the automatic chunk is within 3 % of the fastest.
+        const int n = boxes[0].n(2);
+        if (!gw_groups_ || integrator_ == 11 || boxes.size() > 1 || n > 256) return c;
+        c.variant = n < 112 ? 3 : kDefaultVariant;
+        const TileVariant &t = kVariants[c.variant];
+        const int ty = t.nw * 64 / t.tx * t.ry;
+        const long long xy = (long long)((boxes[0].n(0) + t.tx - 1) / t.tx) *
+                             ((boxes[0].n(1) + ty - 1) / ty);
+        c.tz = 32;
+        while (c.tz > 4 && xy * ((n + c.tz - 1) / c.tz) < 2LL * ncu_) c.tz /= 2;
+        c.tz = std::min(c.tz, n);
+        return c;
+    }
     const int kind = integrator_ == 10 ? kSsprk1 : integrator_ == 11 ? kLeap1 : kRkn0;
     const auto &row = kt_.stage[kind][(int)prec_][R_][0][0];
     int maxn = 1;
@@ -1169,14 +1185,21 @@ LaunchCfg Runtime::rule_launch(const LevelState &ls, int fused) const {
     }
     // Many boxes: enough tiles that the rounds even out, so the shape with
     // the least padding wins (measured weight per padded cell: a 32-wide
-    // plane 1.2x a 64-wide one; 16..64-cell boxes: 2.95 to 2.37 ms for the
-    // three SSPRK3 stages of 39.5 M cells, 32^3..160^3: 1.62 to 1.50 ms per
-    // RKN4 step with two rows per thread), on chunks of 16 planes, or 8
-    // where 16 leave fewer than four tiles per CU.
+    // plane 1.2x a 64-wide one), one tile per workgroup.  Three SSPRK3 stages
+    // of 39.5 M cells in boxes 16..64 wide: 2.95 ms on 64 x 8 tiles of 16
+    // planes, 2.62 on 32 x 8, 2.45 without the persistent walk, 2.38 on 8
+    // planes without the XCD ranges; RKN4 step of boxes 32^3..160^3: 1.62 ms
+    // on 64 x 8, 1.50 with two rows per thread (one field up to radius 2 also
+    // on FP64 tiles of stored pairs: 1.88 to 1.72), 1.41 without the
+    // persistent walk.  Chunks of 16 planes for one field, 8 for more, or
+    // fewer where that leaves less than four tiles per CU.
+    const bool two_rows = kt_.nfields == 1 && (one_field || R_ <= 2);
     double bw = 1e30;
     for (int v = 0; v < kNVar; ++v) {
-        if (!usable(v)) continue;
         const TileVariant &t = kVariants[v];
+        if (!row[v].fn || (t.tx == 32 && R_ >= 3)) continue;
+        // Two rows per thread stand in for the taller 64-wide tiles.
+        if (t.tx == 64 && (two_rows ? t.ry == 1 && t.nw > 4 : t.ry > 1)) continue;
         double planes;
         (void)tiles(t.tx, t.nw * 64 / t.tx * t.ry, std::min(16, maxn), planes);
         const double w = planes * t.nw * t.ry *
@@ -1186,9 +1209,11 @@ LaunchCfg Runtime::rule_launch(const LevelState &ls, int fused) const {
             c.variant = v;
         }
     }
+    c.persistent = 0;
+    c.xcd_split = kt_.nfields == 1 ? 1 : 0;
     const TileVariant &t = kVariants[c.variant];
     double p;
-    c.tz = 16;
+    c.tz = kt_.nfields == 1 ? 16 : 8;
     while (c.tz > 4 && tiles(t.tx, t.nw * 64 / t.tx * t.ry, c.tz, p) < 4LL * ncu_) c.tz /= 2;
     c.tz = std::min(c.tz, maxn);
     return c;

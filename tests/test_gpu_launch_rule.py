@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import sledgehamr_amd as shm
-from cases import complex_scalar, ensemble_inputs, real_scalar
+from cases import complex_scalar, ensemble_inputs, phase_transition, real_scalar
 
 pytestmark = pytest.mark.gpu
 
@@ -57,3 +57,19 @@ def test_ragged_ensembles(edges, prec):
     boxes = [[0, 0, 0, a - 1, b - 1, c - 1] for a, b, c in edges]
     inp = ensemble_inputs([[0, 0, 0, 127, 127, 127]], integrator=21, order=2)
     _same_as_fixed("RealScalar", inp, prec, boxes)
+
+
+@pytest.mark.parametrize("N", [14, 48, 66, 112, 130])
+@pytest.mark.parametrize("integrator", [10, 21])
+@pytest.mark.parametrize("prec", [shm.PREC_FP64, shm.PREC_FP32C16, shm.PREC_FP32CS])
+def test_gw_groups(N, integrator, prec):
+    _same_as_fixed("PhaseTransitionGW", phase_transition(N=N, integrator=integrator, **ANY),
+                   prec, steps=2)
+
+
+@pytest.mark.parametrize("prec", [shm.PREC_FP64, shm.PREC_FP32C16])
+def test_two_fields_in_many_boxes(prec):
+    inp = complex_scalar(N=64, **{"shm.independent_boxes": 1})
+    boxes = [[0, 0, 0, a - 1, b - 1, c - 1] for a, b, c in
+             [(16, 16, 16), (64, 34, 18), (30, 62, 33), (32, 32, 32), (9, 8, 7)] * 4]
+    _same_as_fixed("ComplexScalar", inp, prec, boxes)
