@@ -1067,10 +1067,11 @@ LaunchCfg Runtime::resolved_launch(int lev) const {
  *  as the planes a resident workgroup walks one after the other (rounds of
  *  the grid times the chunk with its R extra queue planes), plus a small
  *  share for the wavefront planes of the whole grid; constants fitted to a
- *  sweep of every shape over 32^3..320^3 levels of one and two fields in
- *  three precisions, where the pick is within 2 % of the fastest shape on
- *  average (default shape 64 x 8 with 16-plane chunks: 25 % on average, 1.55x
- *  at 32^3, where its 4 workgroups walk 16 planes each). */
+ *  sweep of every shape over levels of one and two fields in three
+ *  precisions.  It serves levels that leave CUs idle: two fields at 32^3 take
+ *  41 us a step (76 on the default 64 x 8 tiles of 16 planes, where 8
+ *  workgroups walk 16 planes each), 128^3 82 us (96); levels from 144^3 up
+ *  have a rule of their own below. */
 LaunchCfg Runtime::rule_launch(const LevelState &ls, int fused) const {
     LaunchCfg c;
     c.variant = kDefaultVariant;
@@ -1101,8 +1102,12 @@ LaunchCfg Runtime::rule_launch(const LevelState &ls, int fused) const {
     int maxn = 1;
     for (const Box3 &b : boxes) maxn = std::max(maxn, b.n(2));
     const bool one_field = kt_.nfields == 1 && !tile_lo();
+    // A thread of a 16-wavefront group has 128 registers: not enough for the
+    // queues of several stencil components in FP64 (RKN at 128^3: 208 us
+    // against 102 on 8 wavefronts).
+    const bool usable16 = kt_.nfields == 1 || !(tile_lo() || prec_ == Prec::F64);
     auto usable = [&](int v) {
-        if (!row[v].fn) return false;
+        if (!row[v].fn || (kVariants[v].nw > 8 && !usable16)) return false;
         // Two rows per thread pay where a thread holds one short queue (one
         // stencil component read as stored: 255 against 315 us at 256^3)
         // and cost registers elsewhere (519 against 470 us with two).
@@ -1139,11 +1144,16 @@ LaunchCfg Runtime::rule_launch(const LevelState &ls, int fused) const {
     // Fused first two stages: one workgroup per CU, a chunk costs 3R + 2
     // extra planes.  SSPRK3 on tiles of the stored type: 354 against 469 us
     // at 256^3 (FP32 + bf16), 576 against 805 us (FP64); 97 to 81 us at
-    // 128^3.  RKN: FP64 up to radius 2 only (340 against 382 us at 256^3;
-    // FP32 within 2 % either way, radius 3 slower).  FP64 tiles of stored
-    // pairs, and ensembles (1.57 against 1.42 ms for 64 boxes): slower.
+    // 128^3.  RKN up to radius 2 only: FP64 (one field at 256^3 335 against
+    // 382 us, two fields 690 against 759), and FP32 on large levels, for two
+    // fields (437 against 482 us at 256^3, equal at 200^3) or one at radius 1
+    // (207 against 230; at radius 2 equal at 256^3 and slower below).  FP64
+    // tiles of stored pairs, and ensembles (1.57 against 1.42 ms for 64
+    // boxes): slower.
     const bool pays = boxes.size() == 1 && maxn >= 64 && !tile_lo() &&
-                      (integrator_ == 10 || (prec_ == Prec::F64 && R_ <= 2));
+                      (integrator_ == 10 ||
+                       (R_ <= 2 && (prec_ == Prec::F64 ||
+                                    (maxn >= 224 && (kt_.nfields > 1 || R_ == 1)))));
     if (fused != 0 && fused_possible(ls) && (fused > 0 || pays)) {
         const FusedEntry *frow = fused_row();
         double bc = 1e30;
@@ -1169,6 +1179,24 @@ LaunchCfg Runtime::rule_launch(const LevelState &ls, int fused) const {
         c.fused_variant = bv;
         c.tz = bz;
         c.variant = best_variant(bz);
+        return c;
+    }
+    double planes;
+    const long long ntile32 =
+        boxes.size() == 1 ? tiles(64, 8, std::min(32, maxn), planes) : 0;
+    if (ntile32 >= ncu_) {
+        // A level that gives every CU a tile of 32 planes (144^3 and up): the
+        // model below counts rounds of an occupancy it guesses, and a wrong
+        // guess costs a last round that is nearly empty (one field at radius
+        // 3: 144 us against 116 at 160^3, 575 against 492 at 300^3).
+        // Automatic chunks give every kernel four rounds or more.  Two rows
+        // per thread for one field at radius 1 or in leapfrog from 200^3 up
+        // (172 against 181 us, 105 against 113, equal from 256^3), else 8
+        // wavefronts.
+        c.tz = 0;
+        const bool two = kt_.nfields == 1 && (R_ == 1 || integrator_ == 11) &&
+                         2 * ntile32 >= 5LL * ncu_;
+        c.variant = two && row[4].fn ? 4 : kDefaultVariant;
         return c;
     }
     if (boxes.size() == 1) {
@@ -1200,7 +1228,6 @@ LaunchCfg Runtime::rule_launch(const LevelState &ls, int fused) const {
         if (!row[v].fn || (t.tx == 32 && R_ >= 3)) continue;
         // Two rows per thread stand in for the taller 64-wide tiles.
         if (t.tx == 64 && (two_rows ? t.ry == 1 && t.nw > 4 : t.ry > 1)) continue;
-        double planes;
         (void)tiles(t.tx, t.nw * 64 / t.tx * t.ry, std::min(16, maxn), planes);
         const double w = planes * t.nw * t.ry *
                          (t.tx == 32 ? 1.2 : t.nw == 4 && t.ry == 1 ? 1.1 : t.nw == 16 ? 1.05 : 1.);

@@ -73,3 +73,14 @@ def test_two_fields_in_many_boxes(prec):
     boxes = [[0, 0, 0, a - 1, b - 1, c - 1] for a, b, c in
              [(16, 16, 16), (64, 34, 18), (30, 62, 33), (32, 32, 32), (9, 8, 7)] * 4]
     _same_as_fixed("ComplexScalar", inp, prec, boxes)
+
+
+@pytest.mark.parametrize("project,N,order,integrator,prec", [
+    ("RealScalar", 150, 3, 21, shm.PREC_FP32CS), ("RealScalar", 202, 1, 11, shm.PREC_FP32C16),
+    ("RealScalar", 226, 1, 21, shm.PREC_FP32C), ("ComplexScalar", 226, 2, 21, shm.PREC_FP32C16),
+    ("ComplexScalar", 160, 2, 21, shm.PREC_FP32CS)])
+def test_levels_that_fill_the_chip(project, N, order, integrator, prec):
+    make = real_scalar if project == "RealScalar" else complex_scalar
+    lc = _same_as_fixed(project, make(N=N, order=order, integrator=integrator, **ANY), prec,
+                        steps=2)
+    assert lc["fused"] == (1 if N == 226 else 0)
