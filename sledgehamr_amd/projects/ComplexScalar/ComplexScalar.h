@@ -54,12 +54,11 @@ void Rhs(const amrex::Array4<double>& rhs,
  *  in the complex plane: +1 upward, -1 downward, 0 if the segment meets the
  *  axis at Re <= 0 or not at all.  Half-open in Im, so a corner on the axis
  *  is counted once.  The crossing abscissa (ar bi - br ai) / (bi - ai) is
- *  positive iff the two products compare as below (no division). */
+ *  positive iff the two products compare as below (no division, no branch). */
 AMREX_GPU_HOST_DEVICE AMREX_FORCE_INLINE
 int PositiveAxisCrossing(double ar, double ai, double br, double bi) {
-    if (ai < 0. && bi >= 0.) return ar * bi > ai * br ? 1 : 0;
-    if (ai >= 0. && bi < 0.) return ar * bi < ai * br ? -1 : 0;
-    return 0;
+    const double p = ar * bi, q = ai * br;
+    return ((ai < 0.) & (bi >= 0.) & (p > q)) - ((ai >= 0.) & (bi < 0.) & (p < q));
 }
 
 /** Winding number of psi around the plaquette spanned at (i, j, k) by the
@@ -92,9 +91,13 @@ bool TagCellForRefinement<true>(const amrex::Array4<const double>& state,
         const int i, const int j, const int k, const int lev, const double time,
         const double dt, const double dx, const double* params) {
     if (params[0] == 0.) return false;
-    return PlaquetteWinding(state, i, j, k, 1, 0, 0, 0, 1, 0) != 0 ||
-           PlaquetteWinding(state, i, j, k, 1, 0, 0, 0, 0, 1) != 0 ||
-           PlaquetteWinding(state, i, j, k, 0, 1, 0, 0, 0, 1) != 0;
+    // All three without a branch: almost every cell needs all of them, and a
+    // branch in between keeps the next plaquette's loads from being issued
+    // (or shared) until the previous one is decided.
+    const int xy = PlaquetteWinding(state, i, j, k, 1, 0, 0, 0, 1, 0);
+    const int xz = PlaquetteWinding(state, i, j, k, 1, 0, 0, 0, 0, 1);
+    const int yz = PlaquetteWinding(state, i, j, k, 0, 1, 0, 0, 0, 1);
+    return (xy | xz | yz) != 0;
 }
 
 /** Truncation-error modifiers (params[0] != 0 switches them on): fields
