@@ -271,7 +271,9 @@ int shm_stream_probe(shm_ctx *ctx, unsigned long long bytes, int reps,
 /* Launch shape of the fused stage kernels.  No counterpart in the reference
  * (AMReX picks its own launch bounds): the tile shape and work order of the
  * persistent tile-table launch.  A field of -1 (tile_z: 0) is not set: the
- * tuned value of the level, else the built-in default, applies. */
+ * tuned value of the level applies, else (variant and tile_z both unset and
+ * untuned) the value a rule on box sizes, precision and field count picks,
+ * else the built-in default.  No shape changes a result. */
 typedef struct shm_launch_t {
     int variant;      /* tile shape: 0..2 = 64 x {4, 8, 16} cells per z plane,
                          one row per thread; 3 = 32 x 8 (two rows per
@@ -281,7 +283,8 @@ typedef struct shm_launch_t {
     int persistent;   /* 1: grid = resident capacity; 0: one tile per workgroup */
     int zc_minor;     /* tile order: 0 = z chunk outermost, 1 = between y and x */
     int fused;        /* SSPRK3, or RKN with a first node 0, on levels of
-                         periodic boxes: stages one and two in one launch */
+                         periodic boxes or of boxes that tile the domain:
+                         stages one and two in one launch */
     int fused_variant;/* tile shape of the fused launch (0..2 as variant) */
 } shm_launch_t;
 
