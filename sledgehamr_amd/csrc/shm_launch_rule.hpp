@@ -1,0 +1,241 @@
+// The rule that picks the launch shape of a level nobody tuned.  Host code
+// without HIP, so it can be checked where there is no GPU.
+#pragma once
+
+#include <algorithm>
+#include <vector>
+
+namespace shm {
+
+struct Box3 {
+    int lo[3], hi[3];  // inclusive, global index space of the level
+    int n(int d) const { return hi[d] - lo[d] + 1; }
+    long long vol() const { return (long long)n(0) * n(1) * n(2); }
+};
+
+/** Tile shape variants: NW wavefronts per workgroup, RY rows per thread, TX
+ *  cells in x (tile = TX x (NW * 64 / TX) * RY cells in x/y).  The 32-wide
+ *  tile serves boxes narrower than 64 cells.  The autotuner picks one per
+ *  level. */
+struct TileVariant {
+    int nw, ry, tx;
+};
+constexpr int kNVar = 5;
+constexpr TileVariant kVariants[kNVar] = {
+    {4, 1, 64}, {8, 1, 64}, {16, 1, 64}, {4, 1, 32}, {4, 2, 64}};
+constexpr int kDefaultVariant = 1;
+
+/** Launch shape of the stage kernels.  A field of -1 (tz: 0) is not set: the
+ *  level's tuned value, else the size rule (LaunchRule) applies. */
+struct LaunchCfg {
+    int variant = -1;     // tile shape index into kVariants
+    int tz = 0;           // z-chunk length of a tile (0: automatic)
+    int xcd_split = -1;   // each XCD walks one contiguous range of tiles
+    int persistent = -1;  // grid = resident capacity (1) or one tile per workgroup (0)
+    int zc_minor = -1;    // tile order: z-chunk outermost (0) or innermost (1)
+    int fused = -1;       // SSPRK3 stages one and two in one launch (0/1)
+    int fused_variant = -1;  // tile shape of that launch
+};
+
+/** What the rule looks at: the stored boxes of a level and what is built for
+ *  its project, precision, radius and integrator. */
+struct LaunchRule {
+    const std::vector<Box3> &boxes;
+    int integrator;          // 10 SSPRK3, 11 leapfrog, 20.. RKN
+    int nfields;
+    int R;                   // stencil radius
+    bool f64;                // states are stored in FP64
+    bool tile_lo;            // FP64 tiles of stored pairs
+    bool gw, gw_groups, ko;
+    int ncu;
+    bool can_fuse;           // the first two stages may run in one launch
+    bool stage_built[kNVar]; // tile shapes of the first stage's kernel
+    int fused_ty[kNVar];     // rows of the fused kernel's tile (0: not built)
+
+    LaunchCfg pick(int fused) const;
+};
+
+/** The launch shape the box sizes ask for.  A stage kernel's time is modelled
+ *  as the planes a resident workgroup walks one after the other (rounds of
+ *  the grid times the chunk with its R extra queue planes), plus a small
+ *  share for the wavefront planes of the whole grid; constants fitted to a
+ *  sweep of every shape over levels of one and two fields in three
+ *  precisions.  It serves levels that leave CUs idle: two fields at 32^3 take
+ *  41 us a step (76 on the default 64 x 8 tiles of 16 planes, where 8
+ *  workgroups walk 16 planes each), 128^3 82 us (96); levels from 144^3 up
+ *  have a rule of their own below. */
+inline LaunchCfg LaunchRule::pick(int fused) const {
+    LaunchCfg c;
+    c.variant = kDefaultVariant;
+    c.fused = 0;
+    // Dissipation is built for one tile shape.
+    if (ko || boxes.empty()) return c;
+    if (gw) {
+        // GW levels run as component groups, nine launches a step with few
+        // wavefronts resident each: chunks short enough for two tiles per CU
+        // (32^3..64^3: 250 to 83-100 us per RKN4 step on 32 x 8 tiles of 4
+        // planes, 96^3 246 to 186, 128^3 342 to 310, 192^3 995 to 961).  From
+        // 256^3 up the automatic chunk is within 3 % of the fastest.
+        const int n = boxes[0].n(2);
+        if (!gw_groups || integrator == 11 || boxes.size() > 1 || n > 256) return c;
+        c.variant = n < 112 ? 3 : kDefaultVariant;
+        const TileVariant &t = kVariants[c.variant];
+        const int ty = t.nw * 64 / t.tx * t.ry;
+        const long long xy = (long long)((boxes[0].n(0) + t.tx - 1) / t.tx) *
+                             ((boxes[0].n(1) + ty - 1) / ty);
+        c.tz = 32;
+        while (c.tz > 4 && xy * ((n + c.tz - 1) / c.tz) < 2LL * ncu) c.tz /= 2;
+        c.tz = std::min(c.tz, n);
+        return c;
+    }
+    int maxn = 1;
+    for (const Box3 &b : boxes) maxn = std::max(maxn, b.n(2));
+    const bool one_field = nfields == 1 && !tile_lo;
+    // A thread of a 16-wavefront group has 128 registers: not enough for the
+    // queues of several stencil components in FP64 (RKN at 128^3: 208 us
+    // against 102 on 8 wavefronts).
+    const bool usable16 = nfields == 1 || !(tile_lo || f64);
+    auto usable = [&](int v) {
+        if (!stage_built[v] || (kVariants[v].nw > 8 && !usable16)) return false;
+        // Two rows per thread pay where a thread holds one short queue (one
+        // stencil component read as stored: 255 against 315 us at 256^3)
+        // and cost registers elsewhere (519 against 470 us with two).
+        if (kVariants[v].ry > 1) return one_field;
+        if (one_field && kVariants[v].tx == 64 && kVariants[v].nw > 4) return false;
+        // At radius 3 a 32 x 8 tile's ring has more cells than the tile.
+        return kVariants[v].tx == 64 || R < 3;
+    };
+    auto tiles = [&](int tx, int ty, int z, double &planes) {
+        long long n = 0;
+        planes = 0;
+        for (const Box3 &b : boxes) {
+            const long long xy = (long long)((b.n(0) + tx - 1) / tx) * ((b.n(1) + ty - 1) / ty);
+            const int k = (b.n(2) + z - 1) / z;
+            n += xy * k;
+            planes += (double)xy * (b.n(2) + k * R);
+        }
+        return n;
+    };
+    auto cost = [&](int v, int z) {
+        double planes;
+        const TileVariant &t = kVariants[v];
+        const long long n = tiles(t.tx, t.nw * 64 / t.tx * t.ry, z, planes);
+        const long long slots = (long long)ncu * std::max(1, 12 / t.nw);
+        return (double)((n + slots - 1) / slots) * (z + R) +
+               0.03 * planes * t.nw * t.ry / ncu;
+    };
+    // -1: no shape the rule would take is built.  Eight stencil components in
+    // FP64 at radius 3 leave the 32 x 8 tile alone; such levels keep the
+    // default, for which the launch takes the nearest built shape.
+    auto best_variant = [&](int z) {
+        int bv = -1;
+        for (int v = 0; v < kNVar; ++v)
+            if (usable(v) && (bv < 0 || cost(v, z) < cost(bv, z))) bv = v;
+        return bv;
+    };
+    // Fused first two stages: one workgroup per CU, a chunk costs 3R + 2
+    // extra planes.  SSPRK3 on tiles of the stored type: 354 against 469 us
+    // at 256^3 (FP32 + bf16), 576 against 805 us (FP64); 97 to 81 us at
+    // 128^3.  RKN up to radius 2 only: FP64 (one field at 256^3 335 against
+    // 382 us, two fields 690 against 759), and FP32 on large levels, for two
+    // fields (437 against 482 us at 256^3, equal at 200^3) or one at radius 1
+    // (207 against 230; at radius 2 equal at 256^3 and slower below).  FP64
+    // tiles of stored pairs, and ensembles (1.57 against 1.42 ms for 64
+    // boxes): slower.
+    const bool pays = boxes.size() == 1 && maxn >= 64 && !tile_lo &&
+                      (integrator == 10 ||
+                       (R <= 2 &&
+                        (f64 || (maxn >= 224 && (nfields > 1 || R == 1)))));
+    if (fused != 0 && can_fuse && (fused > 0 || pays)) {
+        double bc = 1e30;
+        int bv = -1, bz = maxn;
+        // The widest tile that still gives half the CUs work at 8 planes.
+        for (int v = kNVar - 1; v >= 0; --v) {
+            double p;
+            if (fused_ty[v] == 0) continue;
+            if (bv < 0 || tiles(64, fused_ty[bv], std::min(8, maxn), p) < ncu / 2) bv = v;
+        }
+        for (int k = 1; k <= maxn; ++k) {
+            const int z = (maxn + k - 1) / k;
+            if (z < 4 && k > 1) break;
+            double p;
+            const long long n = tiles(64, fused_ty[bv], z, p);
+            const double m = (double)((n + ncu - 1) / ncu) * (z + 3 * R + 2);
+            if (m < bc) {
+                bc = m;
+                bz = z;
+            }
+        }
+        c.fused = 1;
+        c.fused_variant = bv;
+        c.tz = bz;
+        if (const int v = best_variant(bz); v >= 0) c.variant = v;
+        return c;
+    }
+    double planes;
+    const long long ntile32 =
+        boxes.size() == 1 ? tiles(64, 8, std::min(32, maxn), planes) : 0;
+    if (ntile32 >= ncu) {
+        // A level that gives every CU a tile of 32 planes (144^3 and up): the
+        // model below counts rounds of an occupancy it guesses, and a wrong
+        // guess costs a last round that is nearly empty (one field at radius
+        // 3: 144 us against 116 at 160^3, 575 against 492 at 300^3).
+        // Automatic chunks give every kernel four rounds or more.  Two rows
+        // per thread for one field at radius 1 or in leapfrog from 200^3 up
+        // (172 against 181 us, 105 against 113, equal from 256^3), else 8
+        // wavefronts.
+        c.tz = 0;
+        const bool two = nfields == 1 && (R == 1 || integrator == 11) &&
+                         2 * ntile32 >= 5LL * ncu;
+        c.variant = two && stage_built[4] ? 4 : kDefaultVariant;
+        return c;
+    }
+    if (boxes.size() == 1) {
+        double bc = 1e30;
+        for (int z = 4; z < 2 * maxn; z *= 2) {
+            const int zz = std::min(z, maxn), v = best_variant(zz);
+            if (v >= 0 && cost(v, zz) < bc) {
+                bc = cost(v, zz);
+                c.variant = v;
+                c.tz = zz;
+            }
+        }
+        return c;
+    }
+    // Many boxes: enough tiles that the rounds even out, so the shape with
+    // the least padding wins (measured weight per padded cell: a 32-wide
+    // plane 1.2x a 64-wide one), one tile per workgroup.  Three SSPRK3 stages
+    // of 39.5 M cells in boxes 16..64 wide: 2.95 ms on 64 x 8 tiles of 16
+    // planes, 2.62 on 32 x 8, 2.45 without the persistent walk, 2.38 on 8
+    // planes without the XCD ranges; RKN4 step of boxes 32^3..160^3: 1.62 ms
+    // on 64 x 8, 1.50 with two rows per thread (one field up to radius 2 also
+    // on FP64 tiles of stored pairs: 1.88 to 1.72), 1.41 without the
+    // persistent walk.  Chunks of 16 planes for one field, 8 for more, or
+    // fewer where that leaves less than four tiles per CU.
+    const bool two_rows = nfields == 1 && (one_field || R <= 2);
+    double bw = 1e30;
+    for (int v = 0; v < kNVar; ++v) {
+        const TileVariant &t = kVariants[v];
+        if (!stage_built[v] || (t.tx == 32 && R >= 3)) continue;
+        // Two rows per thread stand in for the taller 64-wide tiles.
+        if (t.tx == 64 && (two_rows ? t.ry == 1 && t.nw > 4 : t.ry > 1)) continue;
+        (void)tiles(t.tx, t.nw * 64 / t.tx * t.ry, std::min(16, maxn), planes);
+        const double w = planes * t.nw * t.ry *
+                         (t.tx == 32 ? 1.2 : t.nw == 4 && t.ry == 1 ? 1.1 : t.nw == 16 ? 1.05 : 1.);
+        if (w < bw) {
+            bw = w;
+            c.variant = v;
+        }
+    }
+    if (bw == 1e30) return c;
+    c.persistent = 0;
+    c.xcd_split = nfields == 1 ? 1 : 0;
+    const TileVariant &t = kVariants[c.variant];
+    double p;
+    c.tz = nfields == 1 ? 16 : 8;
+    while (c.tz > 4 && tiles(t.tx, t.nw * 64 / t.tx * t.ry, c.tz, p) < 4LL * ncu) c.tz /= 2;
+    c.tz = std::min(c.tz, maxn);
+    return c;
+}
+
+}  // namespace shm

@@ -16,6 +16,7 @@
 #include <utility>
 #include <vector>
 
+#include "shm_launch_rule.hpp"
 #include "shm_layout.hpp"
 #include "shm_stage.hpp"
 #include "shm_table.hpp"
@@ -35,12 +36,6 @@ constexpr size_t kScratchNormOff = 2048;       // level-norm maxima (u64 bits)
 constexpr size_t kScratchRecOff = 2560;        // coarse/fine fill record
 constexpr size_t kScratchMaskOff = 4096;       // tag mask, one byte per cell
 constexpr long long kScratchMaxCells = (long long)(kScratchBytes - kScratchMaskOff);
-
-struct Box3 {
-    int lo[3], hi[3];  // inclusive, global index space of the level
-    int n(int d) const { return hi[d] - lo[d] + 1; }
-    long long vol() const { return (long long)n(0) * n(1) * n(2); }
-};
 
 /** Owning device allocation. */
 class DevMem {
@@ -111,18 +106,6 @@ struct Layout {
                bool is_periodic, bool is_independent = false, bool may_merge = false);
     const TileDesc *get_tiles(int ty, int tz, int zc_minor, int *ntiles, int tx = 64);
     long long nvalid() const { return vprefix.empty() ? 0 : vprefix.back(); }
-};
-
-/** Launch shape of the stage kernels.  A field of -1 (tz: 0) is not set: the
- *  level's tuned value, else the size rule (Runtime::rule_launch) applies. */
-struct LaunchCfg {
-    int variant = -1;     // tile shape index into kVariants
-    int tz = 0;           // z-chunk length of a tile (0: automatic)
-    int xcd_split = -1;   // each XCD walks one contiguous range of tiles
-    int persistent = -1;  // grid = resident capacity (1) or one tile per workgroup (0)
-    int zc_minor = -1;    // tile order: z-chunk outermost (0) or innermost (1)
-    int fused = -1;       // SSPRK3 stages one and two in one launch (0/1)
-    int fused_variant = -1;  // tile shape of that launch
 };
 
 /** Device state of one level: the old/new state pair and stage scratch. */

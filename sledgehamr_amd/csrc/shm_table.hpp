@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "shm_launch_rule.hpp"
 #include "shm_layout.hpp"
 
 namespace shm {
@@ -41,18 +42,6 @@ enum StageKind : int {
     kRknF2Y,       // final stage of a three-stage step reading them
     kNKind
 };
-
-/** Tile shape variants: NW wavefronts per workgroup, RY rows per thread, TX
- *  cells in x (tile = TX x (NW * 64 / TX) * RY cells in x/y).  The 32-wide
- *  tile serves boxes narrower than 64 cells.  The autotuner picks one per
- *  level. */
-struct TileVariant {
-    int nw, ry, tx;
-};
-constexpr int kNVar = 5;
-constexpr TileVariant kVariants[kNVar] = {
-    {4, 1, 64}, {8, 1, 64}, {16, 1, 64}, {4, 1, 32}, {4, 2, 64}};
-constexpr int kDefaultVariant = 1;
 
 using StageFn = hipError_t (*)(const StageArgs &, int grid, hipStream_t);
 using FusedFn = hipError_t (*)(const FusedArgs &, int grid, hipStream_t);
