@@ -828,6 +828,8 @@ void Runtime::init_from_inputs(const std::string &inputs,
     pp.query("shm.independent_boxes", independent_);
     if (independent_ && S.max_level > 0)
         throw Error(1, "shm.independent_boxes needs a single level");
+    // Level-0 boxes that tile the domain as one brick, or box by box.
+    pp.query("shm.merge_boxes", merge_level0_);
     pp.query("shm.tile_order_zc_minor", launch.zc_minor);
     pp.query("shm.graphs", graphs);
     pp.query("shm.fused", launch.fused);
@@ -975,7 +977,8 @@ void Runtime::set_level(int lev, const std::vector<Box3> &boxes) {
             if (b.lo[a] < 0 || b.hi[a] >= N || b.hi[a] < b.lo[a])
                 throw Error(1, "box outside the level domain");
     const bool indep = independent_ && lev == 0;
-    ls.L.build(boxes, sim_->nghost, N, /*periodic=*/!indep, indep, /*may_merge=*/lev == 0);
+    ls.L.build(boxes, sim_->nghost, N, /*periodic=*/!indep, indep,
+               /*may_merge=*/lev == 0 && merge_level0_);
     ls.ncomp = ncomp_;
     ensure_arrays(ls, integrator_);
     ls.t = sim_->t_start;
@@ -2053,7 +2056,7 @@ void Runtime::define_shadow() {
     if (!shadow_.defined() || shadow_.L.boxes.size() != l0.L.boxes.size()) {
         shadow_ = LevelState();
         shadow_.L.build(coarsen(l0.L.boxes), sim_->nghost,
-                        sim_->coarse_level_grid_size / 2, true, false, /*may_merge=*/true);
+                        sim_->coarse_level_grid_size / 2, true, false, merge_level0_);
         shadow_.ncomp = ncomp_;
         ensure_arrays(shadow_, integrator_);
         shadow_.t = l0.t;

@@ -470,6 +470,7 @@ class Runtime {
     bool gw_ = false, ko_ = false;
     int interp_type_ = 2;  // amr.interpolation_type (0 or 2)
     bool independent_ = false;  // level-0 boxes are separate periodic domains
+    bool merge_level0_ = true;  // shm.merge_boxes (Layout::merged)
     std::map<int, std::vector<long long>> last_tags_;
     int integrator_ = 10;
     std::vector<double> nodes_, bbar_, b_;

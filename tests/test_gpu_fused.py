@@ -137,7 +137,7 @@ def test_fused_in_captured_steps():
 def test_multibox_level_keeps_two_launches():
     """Boxes that do not wrap on themselves need ghost cells the fused
     kernel does not have: the level stays on the two-launch path."""
-    inp = dict(complex_scalar(N=32), **{"amr.max_grid_size": 16})
+    inp = dict(complex_scalar(N=32), **{"amr.max_grid_size": 16, "shm.merge_boxes": 0})
     sim = shm.Simulation("ComplexScalar", inp, precision=shm.PREC_FP32C16)
     sim.set_launch(fused=1)
     assert sim.get_launch(0)["fused"] == 0
@@ -265,7 +265,7 @@ def test_rkn_second_stage_state_equals_composed(layout, integrator, prec):
         inp = ensemble_inputs(boxes, integrator=integrator)
         fields = ensemble_fields(boxes, seed=8)
     else:
-        extra = {"amr.max_grid_size": 16} if layout == "boxes" else {}
+        extra = {"amr.max_grid_size": 16, "shm.merge_boxes": 0} if layout == "boxes" else {}
         inp = real_scalar(N=32, order=2, integrator=integrator, lam=1.0, **extra)
         boxes, fields = None, _rkn_fields(32, 3)
     sims = []

@@ -102,13 +102,15 @@ def test_dissipation_damps_high_modes():
     assert energy[True] < 0.1 * e0, energy
 
 
+@pytest.mark.parametrize("merge", [0, 1])
 @pytest.mark.parametrize("prec", [shm.PREC_FP64, shm.PREC_FP32C16, shm.PREC_FP32CS])
-def test_multibox_dissipation_radius3(prec):
-    """Order-3 dissipation over 8 boxes of 16^3 with 3 ghost cells equals
-    the single box bit for bit."""
+def test_multibox_dissipation_radius3(prec, merge):
+    """Order-3 dissipation over 8 boxes of 16^3 with 3 ghost cells (stored box
+    by box, or as one brick) equals the single box bit for bit."""
     base = _inputs(3, integrator=10)
     a = shm.Simulation("RealScalar", base, precision=prec)
-    b = shm.Simulation("RealScalar", dict(base, **{"amr.max_grid_size": 16}),
+    b = shm.Simulation("RealScalar", dict(base, **{"amr.max_grid_size": 16,
+                                                   "shm.merge_boxes": merge}),
                        precision=prec)
     glob = [gaussian_random_field(32, seed=s, kcut=12, std=0.2).reshape(32, 32, 32)
             for s in (5, 6)]

@@ -112,13 +112,15 @@ def test_device_initial_state_matches_oracle():
         assert np.max(np.abs(sim.download(0, c) - orc.download(0, c))) < 1e-13
 
 
+@pytest.mark.parametrize("merge", [0, 1])
 @pytest.mark.parametrize("prec", ALLP)
-def test_multibox_equals_single_box(prec):
-    """A level chopped into 8 boxes (box-to-box halos) gives the single-box
-    result bit-for-bit."""
+def test_multibox_equals_single_box(prec, merge):
+    """A level chopped into 8 boxes, stored box by box (box-to-box halos) or
+    as one brick, gives the single-box result bit-for-bit."""
     base = complex_scalar(N=32, integrator=10)
     a = shm.Simulation("ComplexScalar", base, precision=prec)
-    b = shm.Simulation("ComplexScalar", dict(base, **{"amr.max_grid_size": 16}),
+    b = shm.Simulation("ComplexScalar", dict(base, **{"amr.max_grid_size": 16,
+                                                      "shm.merge_boxes": merge}),
                        precision=prec)
     orc = Oracle("ComplexScalar", base)
     orc.init_state(0, 1, seed=3, params=[0.05])

@@ -22,7 +22,7 @@ NARROW = [[0, 0, 0, 23, 31, 15], [24, 0, 0, 47, 31, 15], [48, 0, 0, 63, 31, 15],
 
 def _run(integrator, prec, variant):
     inp = real_scalar(N=64, order=2, nghost=2, lam=1.0, L=16.0, integrator=integrator,
-                      **{"shm.independent_boxes": 0})
+                      **{"shm.independent_boxes": 0, "shm.merge_boxes": 0})
     sim = shm.Simulation("RealScalar", inp, precision=prec)
     sim.set_boxes(0, NARROW)
     for c, ph in ((0, 0.4), (1, 1.3)):
@@ -49,7 +49,8 @@ def test_tile_variants_agree(integrator, prec):
 
 @pytest.mark.parametrize("prec,tol", [(shm.PREC_FP64, 1e-12)])
 def test_narrow_tile_matches_oracle(prec, tol):
-    inp = real_scalar(N=64, order=2, nghost=2, lam=1.0, L=16.0, integrator=21)
+    inp = real_scalar(N=64, order=2, nghost=2, lam=1.0, L=16.0, integrator=21,
+                      **{"shm.merge_boxes": 0})
     sim = shm.Simulation("RealScalar", inp, precision=prec)
     orc = Oracle("RealScalar", inp)
     for o in (sim, orc):
