@@ -1091,8 +1091,8 @@ const FusedEntry *Runtime::fused_row() const {
 }
 
 /** The first two stages run in one pass: SSPRK3, or RKN whose first node is
- *  0 and which has a third stage, without dissipation, on a level of boxes
- *  that wrap on themselves. */
+ *  0 and which has a third stage, without dissipation, on a level whose
+ *  stored boxes wrap on themselves. */
 bool Runtime::fused_possible(const LevelState &ls) const {
     if (ko_) return false;
     if (integrator_ >= 20) {
@@ -1104,9 +1104,6 @@ bool Runtime::fused_possible(const LevelState &ls) const {
     bool any = false;
     for (int v = 0; v < kNVar; ++v) any = any || row[v].fn != nullptr;
     if (!any) return false;
-    // A merged level (many boxes stored as one brick) keeps separate launches
-    // below 64 cells per axis, where the two are equal within 3 %.
-    if (ls.L.merged && ls.L.N < 64) return false;
     for (const BoxDesc &b : ls.L.hsbox)
         if (b.wrap != 7) return false;
     return !ls.L.hsbox.empty();

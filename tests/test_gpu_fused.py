@@ -134,6 +134,26 @@ def test_fused_in_captured_steps():
     assert b._get_info()["graph_replays"] == 4
 
 
+@pytest.mark.parametrize("project,N", [("ComplexScalar", 32), ("RealScalar", 16)])
+@pytest.mark.parametrize("prec", ALLP)
+def test_fused_on_boxes_that_tile_the_domain(project, N, prec):
+    """A chopped level is stored as one brick, which fuses when asked to, on
+    small levels too."""
+    inp = complex_scalar(N=N) if project == "ComplexScalar" else \
+        real_scalar(N=N, order=2, integrator=21)
+    a, b = _pair(project, dict(inp, **{"amr.max_grid_size": N // 2}), prec, 1)
+    rng = np.random.default_rng(N)
+    nc = a.info["ncomp"]
+    for c in range(nc):
+        d = 0.2 * rng.standard_normal(N ** 3) + (c == 0)
+        a.upload(0, c, d)
+        b.upload(0, c, d)
+    a.advance(0, 3)
+    b.advance(0, 3)
+    assert b.get_launch(0)["fused"] == 1 and a.get_launch(0)["fused"] == 0
+    _same(a, b, 0, nc, ("brick", project, prec))
+
+
 def test_multibox_level_keeps_two_launches():
     """Boxes that do not wrap on themselves need ghost cells the fused
     kernel does not have: the level stays on the two-launch path."""
