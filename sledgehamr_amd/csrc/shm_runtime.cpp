@@ -15,7 +15,6 @@
 #include <hipfft/hipfft.h>
 
 #include <algorithm>
-#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstring>
@@ -27,6 +26,7 @@
 
 #include "shm_aux.hpp"
 #include "shm_fused.hpp"
+#include "shm_to_host.hpp"
 
 // ---------------------------------------------------------------------------
 // ParmParse table.
@@ -435,16 +435,8 @@ __global__ void __launch_bounds__(64) clear_words_kernel(unsigned long long *p, 
 }
 
 // ---------------------------------------------------------------------------
-// Pinned rings of the transfers to the host.  Pinning 32 MB takes milliseconds,
-// so a ring outlives the call and the context that first needed it: calls take
-// one from the process's pool and give it back, the pool keeps at most
-// kIoKeep, and the last context of the process to close frees them.
+// Pinned rings of the transfers to the host (shm_to_host.hpp).
 // ---------------------------------------------------------------------------
-
-constexpr size_t kIoSlot = 8u << 20;   // bytes a producer fills at a time
-constexpr int kIoSlots = 4;
-constexpr size_t kIoUnit = 2u << 20;   // bytes a thread copies at a time
-constexpr size_t kIoKeep = 4;
 
 struct IoRing {
     char *host = nullptr;
@@ -460,64 +452,28 @@ struct IoRing {
     }
 };
 
-class IoPool {
-  public:
-    void enter() {
-        std::lock_guard<std::mutex> lk(mu_);
-        ++users_;
+static IoRing make_ring(size_t bytes, int device) {
+    IoRing r;
+    r.device = device;
+    r.bytes = bytes;
+    try {
+        void *p = nullptr;
+        SHM_HIP(hipHostMalloc(&p, bytes, hipHostMallocDefault));
+        r.host = static_cast<char *>(p);
+        void *d = nullptr;
+        SHM_HIP(hipHostGetDevicePointer(&d, p, 0));
+        r.dev = static_cast<char *>(d);
+        for (hipEvent_t &e : r.ev)
+            SHM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    } catch (...) {
+        r.reset();
+        throw;
     }
-    void leave() {
-        std::lock_guard<std::mutex> lk(mu_);
-        if (--users_ == 0) {
-            for (IoRing &r : free_) r.reset();
-            free_.clear();
-        }
-    }
-    IoRing take(size_t bytes, int device) {
-        bytes = bytes <= kIoUnit ? kIoUnit : kIoSlot * kIoSlots;
-        {
-            std::lock_guard<std::mutex> lk(mu_);
-            for (size_t i = 0; i < free_.size(); ++i)
-                if (free_[i].bytes == bytes && free_[i].device == device) {
-                    const IoRing r = free_[i];
-                    free_.erase(free_.begin() + i);
-                    return r;
-                }
-        }
-        IoRing r;
-        r.device = device;
-        r.bytes = bytes;
-        try {
-            void *p = nullptr;
-            SHM_HIP(hipHostMalloc(&p, bytes, hipHostMallocDefault));
-            r.host = static_cast<char *>(p);
-            void *d = nullptr;
-            SHM_HIP(hipHostGetDevicePointer(&d, p, 0));
-            r.dev = static_cast<char *>(d);
-            for (hipEvent_t &e : r.ev)
-                SHM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        } catch (...) {
-            r.reset();
-            throw;
-        }
-        return r;
-    }
-    void give(IoRing r) {
-        std::lock_guard<std::mutex> lk(mu_);
-        if (users_ > 0 && free_.size() < kIoKeep)
-            free_.push_back(r);
-        else
-            r.reset();
-    }
+    return r;
+}
 
-  private:
-    std::mutex mu_;
-    std::vector<IoRing> free_;
-    int users_ = 0;
-};
-
-static IoPool &io_pool() {
-    static IoPool *p = new IoPool;  // outlives contexts closed at process exit
+static IoPool<IoRing> &io_pool() {
+    static IoPool<IoRing> *p = new IoPool<IoRing>;  // outlives contexts closed at process exit
     return *p;
 }
 
@@ -2343,18 +2299,9 @@ void Runtime::upload_array(int lev, int comp_id, const double *host, int layout)
     upload(lev, comp_id, v.data());
 }
 
-/** Pageable copies by the HIP runtime run at the pace of one thread that
- *  copies out of its staging buffer and takes the page faults of a freshly
- *  allocated array: 9.8 GB/s into numpy memory (13.7 ms for a 256^3
- *  component).  Here (38 GB/s, 3.5 ms) several threads share
- *  both (units of 2 MB of the destination, so two threads rarely fault on
- *  one large page), while the device fills the next slots. */
 void Runtime::to_host(void *dst, size_t nbytes,
                       const std::function<void(size_t, size_t, void *, void *)> &produce) {
     if (nbytes == 0) return;
-    static_assert(kIoSlot % kIoUnit == 0, "slots hold whole units");
-    constexpr size_t kUnit = kIoUnit;
-    char *out = static_cast<char *>(dst);
     struct Lease {
         IoRing r;
         hipStream_t s;
@@ -2363,66 +2310,24 @@ void Runtime::to_host(void *dst, size_t nbytes,
             (void)hipStreamSynchronize(s);
             io_pool().give(r);
         }
-    } lease{io_pool().take(nbytes, device_), stream_};
+    } lease{io_pool().take(nbytes <= kIoUnit ? kIoUnit : kIoSlot * kIoSlots, device_, make_ring),
+            stream_};
     IoRing &ring = lease.r;
-    if (nbytes <= kUnit) {
+    if (nbytes <= kIoUnit) {
         produce(0, nbytes, ring.host, ring.dev);
         SHM_HIP(hipStreamSynchronize(stream_));
-        std::memcpy(out, ring.host, nbytes);
+        std::memcpy(dst, ring.host, nbytes);
         return;
     }
-    const size_t nchunk = (nbytes + kIoSlot - 1) / kIoSlot;
-    const size_t upc = kIoSlot / kUnit;  // units per chunk
-    const size_t nunit = (nbytes + kUnit - 1) / kUnit;
-    std::vector<std::atomic<int>> left(nchunk);  // units of a chunk not copied yet
-    for (size_t c = 0; c < nchunk; ++c)
-        left[c] = (int)(std::min(nunit, (c + 1) * upc) - c * upc);
-    std::atomic<size_t> ready{0}, unit{0};
-    std::atomic<bool> stop{false};
-    auto work = [&] {
-        for (size_t u = unit++; u < nunit; u = unit++) {
-            const size_t c = u / upc;
-            while (ready.load(std::memory_order_acquire) <= c) {
-                if (stop) return;
-                std::this_thread::yield();
-            }
-            const size_t o = u * kUnit, n = std::min(kUnit, nbytes - o);
-            std::memcpy(out + o, ring.host + (c % kIoSlots) * kIoSlot + (o - c * kIoSlot), n);
-            left[c].fetch_sub(1, std::memory_order_release);
-        }
-    };
-    const unsigned hc = std::max(1u, std::thread::hardware_concurrency());
-    const size_t nthr = std::min<size_t>({8, hc, nunit / 2});
-    std::vector<std::thread> thr;
-    struct Join {
-        std::vector<std::thread> &t;
-        std::atomic<bool> &stop;
-        ~Join() {
-            stop = true;
-            for (std::thread &x : t) x.join();
-        }
-    } join{thr, stop};
-    size_t queued = 0;
-    for (size_t c = 0; c < nchunk; ++c) {
-        // Fill every free slot, then wait for chunk c.
-        for (; queued < nchunk && queued < c + kIoSlots; ++queued) {
-            if (queued >= kIoSlots) {
-                const size_t old = queued - kIoSlots;
-                if (left[old].load(std::memory_order_acquire) > 0 && queued > c) break;
-                while (left[old].load(std::memory_order_acquire) > 0) std::this_thread::yield();
-            }
-            const size_t o = queued * kIoSlot;
-            const size_t at = (queued % kIoSlots) * kIoSlot;
-            produce(o, std::min(kIoSlot, nbytes - o), ring.host + at, ring.dev + at);
-            SHM_HIP(hipEventRecord(ring.ev[queued % kIoSlots], stream_));
-        }
-        if (c == 0)
-            for (size_t i = 0; i < nthr; ++i) thr.emplace_back(work);
-        SHM_HIP(hipEventSynchronize(ring.ev[c % kIoSlots]));
-        ready.store(c + 1, std::memory_order_release);
-    }
-    for (std::thread &x : thr) x.join();
-    thr.clear();
+    copy_through_slots(
+        static_cast<char *>(dst), nbytes, ring.host,
+        [&](size_t o, size_t bytes, int slot) {
+            const size_t at = slot * kIoSlot;
+            produce(o, bytes, ring.host + at, ring.dev + at);
+            SHM_HIP(hipEventRecord(ring.ev[slot], stream_));
+        },
+        [&](int slot) { SHM_HIP(hipEventSynchronize(ring.ev[slot])); },
+        [](auto f) { return std::thread(f); });
 }
 
 void Runtime::valid_io(LevelState &ls, int comp_id, int which, double *host, bool to_state) {
