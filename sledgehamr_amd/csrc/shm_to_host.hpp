@@ -8,6 +8,7 @@
 #include <cstddef>
 #include <cstring>
 #include <mutex>
+#include <system_error>
 #include <thread>
 #include <utility>
 #include <vector>
@@ -68,7 +69,8 @@ class IoPool {
 /** Moves nbytes through kIoSlots slots of kIoSlot bytes into out.
  *  produce(offset, bytes, slot) enqueues what writes those bytes into a slot,
  *  wait(slot) returns when they are there, start(f) starts a thread that runs
- *  f.  Pageable copies by the HIP runtime run at the pace of one thread that
+ *  f or throws std::system_error.
+ *  Pageable copies by the HIP runtime run at the pace of one thread that
  *  copies out of its staging buffer and takes the page faults of a freshly
  *  allocated array: 9.8 GB/s into numpy memory (13.7 ms for a 256^3
  *  component).  Here (38 GB/s, 3.5 ms) several threads share both (units of
@@ -86,16 +88,18 @@ void copy_through_slots(char *out, size_t nbytes, const char *slots, Produce &&p
         left[c] = (int)(std::min(nunit, (c + 1) * upc) - c * upc);
     std::atomic<size_t> ready{0}, unit{0};
     std::atomic<bool> stop{false};
+    auto copy_unit = [&](size_t u) {
+        const size_t c = u / upc, o = u * kIoUnit, n = std::min(kIoUnit, nbytes - o);
+        std::memcpy(out + o, slots + (c % kIoSlots) * kIoSlot + (o - c * kIoSlot), n);
+        left[c].fetch_sub(1, std::memory_order_release);
+    };
     auto work = [&] {
         for (size_t u = unit++; u < nunit; u = unit++) {
-            const size_t c = u / upc;
-            while (ready.load(std::memory_order_acquire) <= c) {
+            while (ready.load(std::memory_order_acquire) <= u / upc) {
                 if (stop) return;
                 std::this_thread::yield();
             }
-            const size_t o = u * kIoUnit, n = std::min(kIoUnit, nbytes - o);
-            std::memcpy(out + o, slots + (c % kIoSlots) * kIoSlot + (o - c * kIoSlot), n);
-            left[c].fetch_sub(1, std::memory_order_release);
+            copy_unit(u);
         }
     };
     const unsigned hc = std::max(1u, std::thread::hardware_concurrency());
@@ -124,9 +128,18 @@ void copy_through_slots(char *out, size_t nbytes, const char *slots, Produce &&p
         wait((int)(c % kIoSlots));
         // The threads poll for the next chunk, so they start when the first
         // one is there: before it the device may still run whole steps.
-        if (c == 0)
-            for (size_t i = 0; i < nthr; ++i) thr.push_back(start(work));
+        if (c == 0) {
+            thr.reserve(nthr);
+            try {
+                for (size_t i = 0; i < nthr; ++i) thr.push_back(start(work));
+            } catch (const std::system_error &) {
+                // As many as the system gives.
+            }
+        }
         ready.store(c + 1, std::memory_order_release);
+        // None: the caller copies.
+        if (thr.empty())
+            for (size_t u = c * upc; u < std::min(nunit, (c + 1) * upc); ++u) copy_unit(u);
     }
     for (std::thread &x : thr) x.join();
     thr.clear();

@@ -1,6 +1,7 @@
 """Transfers through rings of slots, on the CPU with slots that a host thread
-fills: every byte arrives whatever the size, and the copying threads take no
-processor time while the device still works on what was queued before."""
+fills: every byte arrives whatever the size and however many threads can be
+started, and the copying threads take no processor time while the device still
+works on what was queued before."""
 import os
 import shutil
 import subprocess
@@ -21,10 +22,11 @@ using namespace shm;
 
 static unsigned char value(size_t i) { return (unsigned char)(i * 2654435761u >> 13); }
 
-// bytes, milliseconds the first slot takes
+// bytes, milliseconds the first slot takes, threads that can be started
 static int transfer(int, char **v) {
     const size_t n = std::strtoull(v[2], nullptr, 10);
     const int ms = std::atoi(v[3]);
+    int threads = std::atoi(v[4]);
     std::vector<char> out(n + 1, 0), slots(kIoSlot * kIoSlots);
     const std::clock_t c0 = std::clock();
     std::clock_t fill = 0;  // the producer's own time
@@ -39,7 +41,12 @@ static int transfer(int, char **v) {
             if (first) std::this_thread::sleep_for(std::chrono::milliseconds(ms));
             first = false;
         },
-        [](auto f) { return std::thread(f); });
+        [&](auto f) {
+            if (threads-- <= 0)
+                throw std::system_error(
+                    std::make_error_code(std::errc::resource_unavailable_try_again));
+            return std::thread(f);
+        });
     const std::clock_t used = std::clock() - c0 - (ms ? fill : 0);
     for (size_t i = 0; i < n; ++i)
         if ((unsigned char)out[i] != value(i)) return std::printf("byte %zu\n", i), 1;
@@ -75,11 +82,12 @@ def exe(tmp_path_factory):
 
 @pytest.mark.parametrize("n", [2 * MIB + 1, 8 * MIB - 1, 8 * MIB, 8 * MIB + 1, 32 * MIB,
                                32 * MIB + 5, 75 * MIB + 3])
-def test_every_byte_arrives(exe, n):
-    exe("transfer", n, 0)
+@pytest.mark.parametrize("threads", [8, 2, 1, 0])
+def test_every_byte_arrives(exe, n, threads):
+    exe("transfer", n, 0, threads)
 
 
 def test_threads_do_not_spin_before_the_first_slot(exe):
     """0.6 s until the first slot is there.  Copying 30 MiB takes some 10 ms of
     processor time; one thread that polls would use 0.6 s."""
-    assert float(exe("transfer", 30 * MIB, 600)[0]) < 0.3
+    assert float(exe("transfer", 30 * MIB, 600, 8)[0]) < 0.3
