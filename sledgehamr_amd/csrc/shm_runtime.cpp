@@ -486,11 +486,10 @@ static IoPool<IoRing> &io_pool() {
 constexpr int kPrmSlots = 1024, kPrmGroup = 8;
 
 Runtime::Runtime(sledgehamr::Sledgehamr *sim, const KernelTable &kt)
-    : sim_(sim), kt_(kt) {
+    : sim_(sim), kt_(kt), io_user_(io_pool()) {
     int dev = 0;
     SHM_HIP(hipGetDevice(&dev));
     device_ = dev;
-    io_pool().enter();
     hipDeviceProp_t prop;
     SHM_HIP(hipGetDeviceProperties(&prop, dev));
     ncu_ = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
@@ -568,7 +567,6 @@ Runtime::~Runtime() {
     if (prm_host_) (void)hipHostFree(prm_host_);
     levels_.clear();
     if (stream_) (void)hipStreamDestroy(stream_);
-    io_pool().leave();
 }
 
 LevelState &Runtime::level(int lev) {

@@ -20,6 +20,7 @@
 #include "shm_layout.hpp"
 #include "shm_stage.hpp"
 #include "shm_table.hpp"
+#include "shm_to_host.hpp"
 
 namespace shm {
 
@@ -107,6 +108,8 @@ struct Layout {
     const TileDesc *get_tiles(int ty, int tz, int zc_minor, int *ntiles, int tx = 64);
     long long nvalid() const { return vprefix.empty() ? 0 : vprefix.back(); }
 };
+
+struct IoRing;  // pinned ring of the transfers to the host
 
 /** Device state of one level: the old/new state pair and stage scratch. */
 struct LevelState {
@@ -422,6 +425,7 @@ class Runtime {
     void to_host(void *dst, size_t nbytes,
                  const std::function<void(size_t, size_t, void *, void *)> &produce);
     int device_ = 0;
+    PoolUser<IoPool<IoRing>> io_user_;
     /** The coarsened copy of level lev (>= 1) on level lev-1, built once
      *  per epoch with its copy plans. */
     LevelState &coarse_mirror(int lev);

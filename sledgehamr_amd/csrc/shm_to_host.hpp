@@ -66,6 +66,20 @@ class IoPool {
     int users_ = 0;
 };
 
+/** A user of a pool for as long as it lives: as a member it leaves the pool
+ *  also when its owner's constructor throws. */
+template <class Pool>
+class PoolUser {
+  public:
+    explicit PoolUser(Pool &p) : p_(p) { p_.enter(); }
+    ~PoolUser() { p_.leave(); }
+    PoolUser(const PoolUser &) = delete;
+    PoolUser &operator=(const PoolUser &) = delete;
+
+  private:
+    Pool &p_;
+};
+
 /** Moves nbytes through kIoSlots slots of kIoSlot bytes into out.
  *  produce(offset, bytes, slot) enqueues what writes those bytes into a slot,
  *  wait(slot) returns when they are there, start(f) starts a thread that runs

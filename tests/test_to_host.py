@@ -1,7 +1,8 @@
 """Transfers through rings of slots, on the CPU with slots that a host thread
 fills: every byte arrives whatever the size and however many threads can be
 started, and the copying threads take no processor time while the device still
-works on what was queued before."""
+works on what was queued before.  The pool frees its rings with its last user,
+also after one whose construction failed."""
 import os
 import shutil
 import subprocess
@@ -55,8 +56,46 @@ static int transfer(int, char **v) {
     return 0;
 }
 
+struct Ring {
+    size_t bytes;
+    int device;
+    int *freed;
+    void reset() { ++*freed; }
+};
+
+struct Context {
+    PoolUser<IoPool<Ring>> user;
+    Context(IoPool<Ring> &p, bool fail) : user(p) {
+        if (fail) throw 1;
+    }
+};
+
+static int pool() {
+    IoPool<Ring> p;
+    int made = 0, freed = 0;
+    auto make = [&](size_t b, int d) { return ++made, Ring{b, d, &freed}; };
+    try {
+        Context c(p, true);
+    } catch (int) {
+    }
+    {
+        Context a(p, false);
+        {
+            Context b(p, false);
+            p.give(p.take(5, 0, make));
+            p.give(p.take(5, 0, make));      // the kept one
+            p.give(p.take(5, 1, make));      // another device
+        }
+        std::printf("%d %d ", made, freed);  // a user is left: kept
+    }
+    std::printf("%d %d ", made, freed);
+    p.give(p.take(5, 0, make));              // no user: not kept
+    std::printf("%d %d\n", made, freed);
+    return 0;
+}
+
 int main(int argc, char **argv) {
-    return transfer(argc, argv);
+    return argc == 2 ? pool() : transfer(argc, argv);
 }
 """
 
@@ -91,3 +130,7 @@ def test_threads_do_not_spin_before_the_first_slot(exe):
     """0.6 s until the first slot is there.  Copying 30 MiB takes some 10 ms of
     processor time; one thread that polls would use 0.6 s."""
     assert float(exe("transfer", 30 * MIB, 600, 8)[0]) < 0.3
+
+
+def test_pool_frees_its_rings_with_its_last_user(exe):
+    assert exe("pool") == ["2", "0", "2", "2", "3", "3"]
