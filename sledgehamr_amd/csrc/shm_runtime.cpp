@@ -2740,6 +2740,10 @@ void Runtime::autotune(int lev) {
     timing_on = false;
     double best = 1e30, best3 = 1e30;
     LaunchCfg bc, bc3;
+    // What the level runs untuned.
+    tuned_[lev + 1] = LaunchCfg();
+    LaunchCfg untuned = resolved_launch(lev);
+    untuned.fused = untuned.fused && fused_possible(ls) ? 1 : 0;
     // Screening times every shape briefly; the few fastest are then timed
     // again at length, since among hundreds of short, noisy timings the
     // smallest is often a mediocre shape that was timed lucky.
@@ -2753,6 +2757,18 @@ void Runtime::autotune(int lev) {
     auto run3 = [&] {
         StageArgs c = s3;
         launch_stage(kSsprk3, ls, c, lev);
+    };
+    // The first two stages in one launch, then the rest of the step.
+    auto run_fused = [&] {
+        launch_fused(ls, prm, prm, dt, lev);
+        if (tune3) {
+            run3();
+        } else {
+            for (size_t k = 2; k < runs.size(); ++k) {
+                StageArgs c = runs[k].second;
+                launch_stage(runs[k].first, ls, c, lev);
+            }
+        }
     };
     for (int v : vs)
         for (int z : zs)
@@ -2814,19 +2830,7 @@ void Runtime::autotune(int lev) {
                 launch.tz = tzc;
                 launch.fused = 1;
                 launch.fused_variant = v;
-                const double ms = time_ms(
-                    [&] {
-                        launch_fused(ls, prm, prm, dt, lev);
-                        if (integrator_ == 10) {
-                            run3();
-                        } else {
-                            for (size_t k = 2; k < runs.size(); ++k) {
-                                StageArgs c = runs[k].second;
-                                launch_stage(runs[k].first, ls, c, lev);
-                            }
-                        }
-                    },
-                    kLongReps);
+                const double ms = time_ms(run_fused, kLongReps);
                 if (ms < best) {
                     best = ms;
                     bc = launch;
@@ -2835,6 +2839,21 @@ void Runtime::autotune(int lev) {
             }
         }
     }
+    // The untuned shape stays where nothing above beats it: the rule knows
+    // chunks that the search leaves out (4 planes: RKN4 at 64^3 27 us a step
+    // on the best shape of the search, 20 on the rule's).  It has as many
+    // tries as the search compares at length, and where a stage takes under
+    // 12 us, the pace at which the host queues them, another shape has to be
+    // faster by a tenth.
+    launch = untuned;
+    double ums = 1e30;
+    for (int i = 0; i < kFinalists; ++i) {
+        double ms = untuned.fused ? time_ms(run_fused, kLongReps) : time_ms(run_all, kLongReps);
+        if (tune3 && !untuned.fused) ms += time_ms(run3, kLongReps);
+        ums = std::min(ums, ms);
+    }
+    const size_t nstage = runs.size() + (tune3 ? 1 : 0);
+    if (ums <= (ums < 0.012 * nstage ? 1.1 : 1.) * best) bc = untuned;
     launch = saved;
     timing_on = saved_t;
     tuned_[lev + 1] = bc;

@@ -2,6 +2,8 @@
 field count picks the tile, the chunk length and whether the first two stages
 run fused): the same cells bit for bit as the 64 x 8 tile on 16-plane chunks
 with separate stages, on sizes at the edges of tiles and chunks."""
+import time
+
 import numpy as np
 import pytest
 
@@ -84,3 +86,31 @@ def test_levels_that_fill_the_chip(project, N, order, integrator, prec):
     lc = _same_as_fixed(project, make(N=N, order=order, integrator=integrator, **ANY), prec,
                         steps=2)
     assert lc["fused"] == (1 if N == 226 else 0)
+
+
+@pytest.mark.parametrize("project,N,integrator,prec", [
+    ("RealScalar", 64, 21, shm.PREC_FP64), ("ComplexScalar", 64, 21, shm.PREC_FP32CS),
+    ("ComplexScalar", 64, 10, shm.PREC_FP64), ("ComplexScalar", 32, 21, shm.PREC_FP32C16),
+    ("RealScalar", 32, 21, shm.PREC_FP32C16)])
+def test_autotuned_level_is_no_slower(project, N, integrator, prec):
+    """The rule's shape is one of the autotuner's candidates.  Without it these
+    levels were 1.26 to 1.38 times slower tuned than untuned; two runs of one
+    shape differ by a few percent."""
+    make = real_scalar if project == "RealScalar" else complex_scalar
+    sim = shm.Simulation(project, make(N=N, integrator=integrator), precision=prec)
+    sim.init_state(0, 1, 3, [0.05])
+
+    def step_time():
+        best = 1e9
+        for _ in range(7):
+            sim.advance(0, 5)
+            sim.sync()
+            t = time.perf_counter()
+            sim.advance(0, 100)
+            sim.sync()
+            best = min(best, time.perf_counter() - t)
+        return best
+    untuned = step_time()
+    sim.autotune(0)
+    tuned = step_time()
+    assert tuned < 1.15 * untuned, (tuned, untuned)
