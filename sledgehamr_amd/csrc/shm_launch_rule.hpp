@@ -169,7 +169,12 @@ inline LaunchCfg LaunchRule::pick(int fused) const {
         c.fused = 1;
         c.fused_variant = bv;
         c.tz = bz;
-        if (const int v = best_variant(bz); v >= 0) c.variant = v;
+        // The remaining stages take the chunk of the fused pass.  Several
+        // components in FP64: eight rows unless it is the shortest (RKN4 of
+        // two fields 306 us unfused, 324 with the model's 64 x 4 and 298 with
+        // 64 x 8 at 176^3; 743 to 662 at 256^3, 53 to 50 at 80^3).
+        const int v = best_variant(bz);
+        if (v >= 0 && (usable16 || bz <= 4)) c.variant = v;
         return c;
     }
     double planes;
@@ -199,6 +204,17 @@ inline LaunchCfg LaunchRule::pick(int fused) const {
                 c.variant = v;
                 c.tz = zz;
             }
+        }
+        // The model counts a plane of a 64 x 4 tile like one of 64 x 8, but
+        // with its ring the first loads 2.1 cells per cell (radius 2), the
+        // second 1.6: on 16 planes, where that is most of the work, several
+        // components in FP64 are faster on the default (112^3 two fields in
+        // FP32CS: RKN4 104 against 90 us, SSPRK3 107 against 93; 128^3 108
+        // against 102 and 108 against 99).  Shorter chunks are not (104^3 82
+        // against 85 us).
+        if (!usable16 && c.variant == 0 && c.tz >= 16) {
+            c.variant = kDefaultVariant;
+            c.tz = 0;
         }
         return c;
     }

@@ -84,3 +84,25 @@ def test_no_usable_shape_leaves_the_default(pick, mask):
     """Eight fields at radius 3 in FP64: nothing, or the 32 x 8 tile alone."""
     cases = [(10, 8, 3, 1, 0, 0, 0, 0, 0, mask, 0, -1, [(n, n, n)]) for n in (16, 64, 128)]
     assert all(r[:2] == (DEFAULT, 0) for r in pick(cases))
+
+
+@pytest.mark.parametrize("integrator,prec", [(10, 3), (21, 3), (11, 3), (11, 0)])
+def test_two_fields_in_fp64_keep_eight_rows(pick, integrator, prec):
+    """112^3 to 128^3: chunks of 16 planes on 64 x 4 tiles, which load 2.1
+    cells per cell at radius 2, took up to 1.15 times as long as the default."""
+    def shape(n):
+        return pick([(integrator, 2, 2, prec == 0, prec == 3, 0, 0, 0, 0, 31, 0, -1,
+                      [(n, n, n)])])[0][:2]
+    assert [shape(n) for n in (112, 120, 128)] == [(DEFAULT, 0)] * 3
+    assert shape(48) == (0, 4) and shape(96) == (3, 8) and shape(136) == (3, 16)
+
+
+@pytest.mark.parametrize("integrator", [10, 21])
+def test_two_fields_in_fp64_keep_eight_rows_beside_the_fused_pass(pick, integrator):
+    """The later stages of a fused FP64 step: 64 x 8 but for 4-plane chunks
+    (176^3 on 64 x 4 tiles was slower than unfused)."""
+    def shape(n):
+        return pick([(integrator, 2, 2, 1, 0, 0, 0, 0, 1, 31, 7, -1, [(n, n, n)])])[0]
+    for n in (80, 112, 142, 176, 256):
+        assert shape(n)[0] == DEFAULT and shape(n)[2] == 1
+    assert shape(64)[1] == 4 and shape(64)[0] != DEFAULT
