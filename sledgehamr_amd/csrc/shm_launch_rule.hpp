@@ -37,6 +37,20 @@ struct LaunchCfg {
     int fused_variant = -1;  // tile shape of that launch
 };
 
+/** z-chunk length for which nothing is set: enough tiles to fill every CU
+ *  several times, long z runs otherwise. */
+inline int auto_chunk(const std::vector<Box3> &boxes, int tx, int ty, int ncu) {
+    int maxn = 1;
+    long long xy = 0;
+    for (const Box3 &b : boxes) {
+        maxn = std::max(maxn, b.n(2));
+        xy += (long long)((b.n(0) + tx - 1) / tx) * ((b.n(1) + ty - 1) / ty);
+    }
+    int z = maxn;
+    while (z > 16 && xy * ((maxn + z - 1) / z) < 8LL * ncu) z = (z + 1) / 2;
+    return z;
+}
+
 /** What the rule looks at: the stored boxes of a level and what is built for
  *  its project, precision, radius and integrator. */
 struct LaunchRule {
@@ -62,7 +76,7 @@ struct LaunchRule {
  *  sweep of every shape over levels of one and two fields in three
  *  precisions.  It serves levels that leave CUs idle: two fields at 32^3 take
  *  41 us a step (76 on the default 64 x 8 tiles of 16 planes, where 8
- *  workgroups walk 16 planes each), 128^3 82 us (96); levels from 144^3 up
+ *  workgroups walk 16 planes each), 128^3 82 us (96); levels from 130^3 up
  *  have a rule of their own below. */
 inline LaunchCfg LaunchRule::pick(int fused) const {
     LaunchCfg c;
@@ -180,8 +194,20 @@ inline LaunchCfg LaunchRule::pick(int fused) const {
     double planes;
     const long long ntile32 =
         boxes.size() == 1 ? tiles(64, 8, std::min(32, maxn), planes) : 0;
-    if (ntile32 >= ncu) {
-        // A level that gives every CU a tile of 32 planes (144^3 and up): the
+    bool fills = ntile32 >= ncu;
+    if (!fills && 8 * ntile32 >= 7LL * ncu) {
+        // One tile short of that (129^3 to 136^3, 255 tiles): on the model's
+        // 16-plane chunks of 32 x 8 tiles one field takes up to 1.27 times as
+        // long as on automatic chunks (RKN4 at radius 3 in FP64 108 against 85
+        // us at 134^3), and so do two fields as long as the automatic chunks
+        // are resident at once (FP32 + bf16 RKN4 128 against 109 us at 134^3;
+        // 130 against 134 at 136^3, where they are not; FP64 leapfrog 79
+        // against 82 at 134^3).
+        const int z = auto_chunk(boxes, 64, 8, ncu);
+        fills = nfields == 1 || (!f64 && tiles(64, 8, z, planes) <= 3LL * ncu);
+    }
+    if (fills) {
+        // A level that gives every CU a tile of 32 planes (138^3 and up): the
         // model below counts rounds of an occupancy it guesses, and a wrong
         // guess costs a last round that is nearly empty (one field at radius
         // 3: 144 us against 116 at 160^3, 575 against 492 at 300^3).

@@ -1140,18 +1140,7 @@ void Runtime::launch_stage(int kind, LevelState &ls, StageArgs &a, int lev) {
         if (gr[0][v].fn && gr[1][v].fn && gr[2][v].fn)
             for (int g = 0; g < 3; ++g) grp[g] = &gr[g][v];
     }
-    int z = lc.tz;
-    if (z <= 0) {
-        // Enough tiles to fill every CU several times, long z runs otherwise.
-        int maxn = 1;
-        long long xy = 0;
-        for (const Box3 &b : ls.L.sboxes) {
-            maxn = std::max(maxn, b.n(2));
-            xy += (long long)((b.n(0) + e.tx - 1) / e.tx) * ((b.n(1) + e.ty - 1) / e.ty);
-        }
-        z = maxn;
-        while (z > 16 && xy * ((maxn + z - 1) / z) < 8LL * ncu_) z = (z + 1) / 2;
-    }
+    const int z = lc.tz > 0 ? lc.tz : auto_chunk(ls.L.sboxes, e.tx, e.ty, ncu_);
     int ntiles = 0;
     a.tiles = ls.L.get_tiles(e.ty, z, lc.zc_minor, &ntiles, e.tx);
     a.boxes = ls.L.dsbox.as<BoxDesc>();

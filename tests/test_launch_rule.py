@@ -106,3 +106,22 @@ def test_two_fields_in_fp64_keep_eight_rows_beside_the_fused_pass(pick, integrat
     for n in (80, 112, 142, 176, 256):
         assert shape(n)[0] == DEFAULT and shape(n)[2] == 1
     assert shape(64)[1] == 4 and shape(64)[0] != DEFAULT
+
+
+def test_levels_just_short_of_filling_the_chip(pick):
+    """130^3 to 136^3 are 255 tiles of 32 planes: chunks of 16 planes took up to
+    1.27 times as long as automatic ones."""
+    def shape(nf, R, integrator, prec, n):
+        return pick([(integrator, nf, R, prec == 0, prec == 3, 0, 0, 0, 0, 31, 0, -1,
+                      [(n, n, n)])])[0][:2]
+    for n in (130, 132, 134):
+        for prec in (1, 2, 3):
+            for R in (1, 2, 3):
+                assert shape(1, R, 21, prec, n) == (DEFAULT, 0)
+                assert shape(1, R, 11, prec, n) == (DEFAULT, 0)
+            assert shape(2, 2, 21, prec, n) == (DEFAULT, 0)
+        assert shape(2, 2, 11, 0, n) == (3, 16)
+    assert shape(1, 3, 21, 0, 136) == (DEFAULT, 0)
+    assert shape(2, 2, 21, 2, 136) == (3, 16)
+    # A corner of the chip stays to the model.
+    assert shape(1, 2, 21, 2, 128)[1] == 8
