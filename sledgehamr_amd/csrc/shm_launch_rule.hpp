@@ -84,24 +84,6 @@ inline LaunchCfg LaunchRule::pick(int fused) const {
     c.fused = 0;
     // Dissipation is built for one tile shape.
     if (ko || boxes.empty()) return c;
-    if (gw) {
-        // GW levels run as component groups, nine launches a step with few
-        // wavefronts resident each: chunks short enough for two tiles per CU
-        // (32^3..64^3: 250 to 83-100 us per RKN4 step on 32 x 8 tiles of 4
-        // planes, 96^3 246 to 186, 128^3 342 to 310, 192^3 995 to 961).  From
-        // 256^3 up the automatic chunk is within 3 % of the fastest.
-        const int n = boxes[0].n(2);
-        if (!gw_groups || integrator == 11 || boxes.size() > 1 || n > 256) return c;
-        c.variant = n < 112 ? 3 : kDefaultVariant;
-        const TileVariant &t = kVariants[c.variant];
-        const int ty = t.nw * 64 / t.tx * t.ry;
-        const long long xy = (long long)((boxes[0].n(0) + t.tx - 1) / t.tx) *
-                             ((boxes[0].n(1) + ty - 1) / ty);
-        c.tz = 32;
-        while (c.tz > 4 && xy * ((n + c.tz - 1) / c.tz) < 2LL * ncu) c.tz /= 2;
-        c.tz = std::min(c.tz, n);
-        return c;
-    }
     int maxn = 1;
     for (const Box3 &b : boxes) maxn = std::max(maxn, b.n(2));
     const bool one_field = nfields == 1 && !tile_lo;
@@ -130,6 +112,49 @@ inline LaunchCfg LaunchRule::pick(int fused) const {
         }
         return n;
     };
+    if (gw) {
+        // GW levels run as three component groups per stage; a group's time is
+        // rounds of its resident workgroups times the chunk with its extra
+        // planes.  FP64 tiles: the groups are built with 4 wavefronts and hold
+        // three workgroups per CU.  FP32: one, three and four, and the three
+        // groups weigh as fitted; the default stays where nothing is 3 %
+        // better.  Over 27 sizes from 32^3 to 256^3, SSPRK3, RKN4 and RKN5,
+        // the pick is within 1 % (FP64) and 2 % of the fastest of 20 shapes on
+        // average and never more than 3 % behind automatic chunks on 64 x 8
+        // tiles, which take 2.2 to 3.4 times as long at 32^3, 1.1 to 1.3 at 96^3,
+        // and are the fastest at 104^3 to 120^3 (chunks of 4 or 8 planes there:
+        // up to 1.27 times as long).
+        const int n = boxes[0].n(2);
+        if (!gw_groups || integrator == 11 || boxes.size() > 1 || n > 256) return c;
+        const bool wide = tile_lo || f64;
+        auto group_cost = [&](int v, int z) {
+            double planes;
+            const TileVariant &t = kVariants[v];
+            const long long nt = tiles(t.tx, t.nw * 64 / t.tx * t.ry, z, planes);
+            auto rounds = [&](int per_cu) {
+                return (double)((nt + (long long)per_cu * ncu - 1) / ((long long)per_cu * ncu));
+            };
+            if (wide) return rounds(3) * (z + 5) + 0.03 * planes * t.nw / ncu;
+            return (v == 3 ? 2.25 * rounds(1) + 1.05 * rounds(3) + 2.8 * rounds(4)
+                           : 4.8 * rounds(1) + 1.8 * rounds(3) + 0.9 * rounds(4)) * (z + 3);
+        };
+        auto chunk = [&](int v, int z) {
+            const TileVariant &t = kVariants[v];
+            return std::min(n, z > 0 ? z : auto_chunk(boxes, t.tx, t.nw * 64 / t.tx * t.ry, ncu));
+        };
+        c.variant = wide ? 0 : kDefaultVariant;
+        const double keep = group_cost(c.variant, chunk(c.variant, 0)) * (wide ? 1. : 0.97);
+        double bc = keep;
+        for (int v : {wide ? 0 : kDefaultVariant, 3})
+            for (int z : {0, 4, 8, 16, 32})
+                if (const double m = group_cost(v, chunk(v, z)); m < bc) {
+                    bc = m;
+                    c.variant = v;
+                    c.tz = chunk(v, z);
+                }
+        if (bc == keep) c.variant = kDefaultVariant;
+        return c;
+    }
     auto cost = [&](int v, int z) {
         double planes;
         const TileVariant &t = kVariants[v];

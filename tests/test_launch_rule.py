@@ -125,3 +125,23 @@ def test_levels_just_short_of_filling_the_chip(pick):
     assert shape(2, 2, 21, 2, 136) == (3, 16)
     # A corner of the chip stays to the model.
     assert shape(1, 2, 21, 2, 128)[1] == 8
+
+
+def _gw(pick, integrator, prec, n):
+    return pick([(integrator, 1, 3, prec == 0, prec == 3, 1, 1, 0, 0, 31, 0, -1,
+                  [(n, n, n)])])[0][:2]
+
+
+@pytest.mark.parametrize("integrator", [10, 21, 22])
+@pytest.mark.parametrize("prec", [0, 1, 2, 3])
+def test_gw_levels(pick, integrator, prec):
+    """Chunks of 4 planes up to 64^3; at 110^3 to 120^3, where short chunks took
+    up to 1.27 times as long, and above 256^3 the automatic ones."""
+    for n in (32, 48, 64):
+        assert _gw(pick, integrator, prec, n)[1] == 4
+    for n in (110, 112, 120, 272, 384):
+        v, z = _gw(pick, integrator, prec, n)
+        assert v in (0, DEFAULT) and (z == 0 or z >= 14)
+    for n in range(8, 258, 2):
+        v, z = _gw(pick, integrator, prec, n)
+        assert v in (0, DEFAULT, 3) and 0 <= z <= n
