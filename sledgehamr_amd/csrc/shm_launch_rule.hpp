@@ -269,39 +269,47 @@ inline LaunchCfg LaunchRule::pick(int fused) const {
         }
         return c;
     }
-    // Many boxes: enough tiles that the rounds even out, so the shape with
-    // the least padding wins (measured weight per padded cell: a 32-wide
-    // plane 1.2x a 64-wide one), one tile per workgroup.  Three SSPRK3 stages
-    // of 39.5 M cells in boxes 16..64 wide: 2.95 ms on 64 x 8 tiles of 16
-    // planes, 2.62 on 32 x 8, 2.45 without the persistent walk, 2.38 on 8
-    // planes without the XCD ranges; RKN4 step of boxes 32^3..160^3: 1.62 ms
-    // on 64 x 8, 1.50 with two rows per thread (one field up to radius 2 also
-    // on FP64 tiles of stored pairs: 1.88 to 1.72), 1.41 without the
-    // persistent walk.  Chunks of 16 planes for one field, 8 for more, or
-    // fewer where that leaves less than four tiles per CU.
-    const bool two_rows = nfields == 1 && (one_field || R <= 2);
+    // Many boxes: the chunk by the cells a CU gets, the shape with the least
+    // padding.  From a sweep of 48 shapes over 220 layouts of 2 to 64 boxes of
+    // 12^3 to 150^3 cells, six of all projects, integrators and precisions
+    // each (1320 levels): the pick is 3 % behind the fastest of the 48 on
+    // average and 15 % faster than 64 x 8 tiles on automatic chunks (41 levels
+    // are 3 to 13 % slower, near the cuts).  A thread with short queues (one
+    // field at radius 1, or in stored FP32 but for SSPRK3) takes two rows, and
+    // chunks of 4 planes up to 3.1 M cells (from 2.0 to 2.7 M 1.02 of the
+    // fastest on average, 8 planes 1.05).  The others keep automatic chunks of
+    // 64 x 8 tiles from 2.1 to 3.1 M cells, where 4, 8 and those are within
+    // 3 % on average and single levels up to 1.17 behind, but FP64, where 8
+    // planes of 32 x 8 are ahead from 1.6 M cells on (1.03 of the fastest,
+    // 64 x 8 1.06).  Weights per padded cell: what 64 x 8 tiles may pad more
+    // and still be as fast.  Large levels of two fields in stored FP32 run
+    // without the XCD ranges (39.5 M cells in boxes 16..64 wide: 2.38 against
+    // 2.45 ms for three SSPRK3 stages), all others with them (FP64: up to 1.36
+    // times as long without).
+    long long cells = 0;
+    for (const Box3 &b : boxes) cells += b.vol();
+    const long long k = cells / (1024LL * ncu);
+    const bool light = nfields == 1 && (R == 1 || (!f64 && !tile_lo && integrator != 10));
+    c.persistent = k < 24 ? 1 : 0;
+    c.xcd_split = nfields > 1 && !f64 && !tile_lo && k >= 56 ? 0 : 1;
+    if (!light && !f64 && k >= 8 && k < 12) return c;
+    c.tz = k < (light ? 12 : f64 ? 6 : 8) ? 4 : k >= 56 && nfields == 1 && R > 1 ? 16 : 8;
+    c.tz = std::min(c.tz, maxn);
+    const double weight[kNVar] = {light ? 1. : 1.08, 1., 0.,
+                                  light ? (f64 ? 1.05 : 1.2) : !f64 ? 1.3 : R < 3 ? 1. : 1.15,
+                                  light ? 0.9 : 1.};
     double bw = 1e30;
     for (int v = 0; v < kNVar; ++v) {
         const TileVariant &t = kVariants[v];
-        if (!stage_built[v] || (t.tx == 32 && R >= 3)) continue;
-        // Two rows per thread stand in for the taller 64-wide tiles.
-        if (t.tx == 64 && (two_rows ? t.ry == 1 && t.nw > 4 : t.ry > 1)) continue;
-        (void)tiles(t.tx, t.nw * 64 / t.tx * t.ry, std::min(16, maxn), planes);
-        const double w = planes * t.nw * t.ry *
-                         (t.tx == 32 ? 1.2 : t.nw == 4 && t.ry == 1 ? 1.1 : t.nw == 16 ? 1.05 : 1.);
+        if (!stage_built[v] || weight[v] == 0.) continue;
+        (void)tiles(t.tx, t.nw * 64 / t.tx * t.ry, c.tz, planes);
+        const double w = planes * t.nw * t.ry * weight[v];
         if (w < bw) {
             bw = w;
             c.variant = v;
         }
     }
-    if (bw == 1e30) return c;
-    c.persistent = 0;
-    c.xcd_split = nfields == 1 ? 1 : 0;
-    const TileVariant &t = kVariants[c.variant];
-    double p;
-    c.tz = nfields == 1 ? 16 : 8;
-    while (c.tz > 4 && tiles(t.tx, t.nw * 64 / t.tx * t.ry, c.tz, p) < 4LL * ncu) c.tz /= 2;
-    c.tz = std::min(c.tz, maxn);
+    if (bw == 1e30) c = LaunchCfg{kDefaultVariant, 0, -1, -1, -1, 0, -1};
     return c;
 }
 

@@ -145,3 +145,19 @@ def test_gw_levels(pick, integrator, prec):
     for n in range(8, 258, 2):
         v, z = _gw(pick, integrator, prec, n)
         assert v in (0, DEFAULT, 3) and 0 <= z <= n
+
+
+def _many(pick, nf, R, integrator, prec, boxes):
+    return pick([(integrator, nf, R, prec == 0, prec == 3, 0, 0, 0, 0, 31, 0, -1, boxes)])[0][:2]
+
+
+def test_many_boxes(pick):
+    """Two fields in boxes 100 wide on 32-wide tiles took up to 1.45 times as
+    long as on the default; boxes 32 wide do need them."""
+    for prec in (1, 2, 3):
+        assert _many(pick, 2, 2, 21, prec, [(100, 100, 100)] * 8) == (DEFAULT, 8)
+        assert _many(pick, 2, 2, 21, prec, [(64, 70, 90)] * 7) == (DEFAULT, 0)
+        assert _many(pick, 2, 2, 10, prec, [(32, 32, 32)] * 1000)[0] == 3
+    assert _many(pick, 2, 2, 21, 0, [(90, 90, 90)] * 8) == (3, 8)
+    assert _many(pick, 1, 2, 21, 2, [(128, 128, 128)] * 32) == (4, 16)
+    assert _many(pick, 1, 1, 21, 2, [(64, 64, 64)] * 8) == (4, 4)
