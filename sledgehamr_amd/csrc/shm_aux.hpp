@@ -389,7 +389,8 @@ struct Walk3 {
  *  thread per parent forms its interpolation coefficients once and writes
  *  its children.
  *
- *  What bounds it: waiting.  A shell tile is small (at most 256 parents) and
+ *  What bounds it: waiting.  A shell tile is small (at most 512 parents of a
+ *  slab one or two parents thick, two passes of the workgroup) and
  *  its work a chain of load, barrier, LDS reads, stores; the values written
  *  (1.05 GB for 22 M ghost cells of a level of 2000 boxes) take 0.2 ms at the
  *  memory rate.  So the chain is kept short: the coarse cell of each of a
@@ -398,7 +399,8 @@ struct Walk3 {
  *  coefficients are formed per parent, not per child (24 children values of
  *  19 LDS reads each were 456 reads, now 57); the two x children of a parent
  *  leave in one store; thin slabs have tiles that are long in their plane
- *  (a 1 x 8 x 4 tile kept 32 of 256 threads busy).  A coarse step of the
+ *  (an x slab one parent thick: 1 x 16 x 8, half of the threads; 1 x 8 x 4
+ *  kept 32 of 256 busy).  A coarse step of the
  *  256^3 base with two levels of 2000 boxes: 43.0 to 33.6 ms. */
 template <Prec P, int MODE, int INTERP>
 __global__ void __launch_bounds__(256) cf_fill_kernel(const CfArgs a) {

@@ -121,9 +121,9 @@ inline LaunchCfg LaunchRule::pick(int fused) const {
         // better.  Over 27 sizes from 32^3 to 256^3, SSPRK3, RKN4 and RKN5,
         // the pick is within 1 % (FP64) and 2 % of the fastest of 20 shapes on
         // average and never more than 3 % behind automatic chunks on 64 x 8
-        // tiles, which take 2.2 to 3.4 times as long at 32^3, 1.1 to 1.3 at 96^3,
-        // and are the fastest at 104^3 to 120^3 (chunks of 4 or 8 planes there:
-        // up to 1.27 times as long).
+        // tiles (7 % over 40 other sizes).  Those take 2.2 to 3.4 times as
+        // long at 32^3, 1.1 to 1.3 at 96^3, and are the fastest at 110^3 to
+        // 120^3 (chunks of 4 or 8 planes there: up to 1.27 times as long).
         const int n = boxes[0].n(2);
         if (!gw_groups || integrator == 11 || boxes.size() > 1 || n > 256) return c;
         const bool wide = tile_lo || f64;

@@ -1363,10 +1363,10 @@ void Runtime::build_cf(int lev) {
     upload_vec(ls.dcf_full, ls.cf_full);
     upload_vec(ls.dcf_step, ls.cf_step);
     // Workgroup tiles: at most 32 x 8 x 4 parents (16 x 8 x 4 for the
-    // quartic's reach 2) of a whole box, and as many as a workgroup has
-    // threads of a shell slab one or two parents thick, long in its plane;
-    // the brick of a tile, its parents grown by the reach, stays within
-    // kCfBrick cells.
+    // quartic's reach 2) of a whole box or a thick slab; of a shell slab one
+    // or two parents thick 256 to 512 (x slabs 128 or 256) that lie long in
+    // its plane, half as many for the quartic's y and z slabs; the brick of a
+    // tile, its parents grown by the reach, stays within kCfBrick cells.
     auto tile = [s](const std::vector<CfPSeg> &v, DevMem &d, int &n, int &lds) {
         std::vector<CfTile> t;
         lds = 0;

@@ -321,8 +321,9 @@ class Runtime {
     /** Launch shape by the level's box sizes alone (nothing timed); fused: 0
      *  or 1 fixes whether the first two stages run in one launch. */
     LaunchCfg rule_launch(const LevelState &ls, int fused) const;
-    /** Fused SSPRK3 stages one and two possible at this level (every box
-     *  periodic on itself, kernel built for the precision and radius). */
+    /** Stages one and two can run in one launch at this level: SSPRK3, or RKN
+     *  with a first node 0, every stored box periodic on itself, kernel built
+     *  for the precision and radius. */
     bool fused_possible(const LevelState &ls) const;
     const FusedEntry *fused_row() const;  // fused12 or fusedrkn, by integrator
 
@@ -352,8 +353,7 @@ class Runtime {
         return tile_lo() ? ls.Ulo[which].get() : nullptr;
     }
     void launch_stage(int pol, LevelState &ls, StageArgs &a, int lev);
-    /** Fused SSPRK3 stages one and two possible at this level (every box
-     *  periodic on itself, kernel built for the precision and radius). */
+    /** Stages one and two in one launch: k2 of SSPRK3, or F0 and F1 of RKN. */
     void launch_fused(LevelState &ls, const double *prm1, const double *prm2,
                       double dt, int lev);
     /** Same-level ghosts of state slot `which`: the leading words, and the
