@@ -173,12 +173,13 @@ inline LaunchCfg LaunchRule::pick(int fused) const {
         return bv;
     };
     // Fused first two stages: one workgroup per CU, a chunk costs 3R + 2
-    // extra planes.  SSPRK3 on tiles of the stored type: 354 against 469 us
-    // at 256^3 (FP32 + bf16), 576 against 805 us (FP64); 97 to 81 us at
-    // 128^3.  RKN up to radius 2 only: FP64 (one field at 256^3 335 against
-    // 382 us, two fields 690 against 759), and FP32 on large levels, for two
-    // fields (437 against 482 us at 256^3, equal at 200^3) or one at radius 1
-    // (207 against 230; at radius 2 equal at 256^3 and slower below).  FP64
+    // extra planes.  Against separate stages on the default shape: SSPRK3 on
+    // tiles of the stored type, two fields, 342 against 492 us at 256^3 (FP32
+    // + bf16), 563 against 899 us (FP64), 65 against 89 and 89 against 120 at
+    // 128^3.  RKN up to radius 2 only: FP64 (one field at 256^3 326 against
+    // 394 us, two fields 662 against 826), and FP32 on large levels, for two
+    // fields (415 against 493 us at 256^3, equal at 200^3) or one at radius 1
+    // (214 against 243; at radius 2 equal at 256^3 and slower below).  FP64
     // tiles of stored pairs, and ensembles (1.57 against 1.42 ms for 64
     // boxes): slower.
     const bool pays = boxes.size() == 1 && maxn >= 64 && !tile_lo &&
