@@ -75,8 +75,8 @@ struct LaunchRule {
  *  share for the wavefront planes of the whole grid; constants fitted to a
  *  sweep of every shape over levels of one and two fields in three
  *  precisions.  It serves levels that leave CUs idle: two fields at 32^3 take
- *  41 us a step (76 on the default 64 x 8 tiles of 16 planes, where 8
- *  workgroups walk 16 planes each), 128^3 82 us (96); levels from 130^3 up
+ *  25 us per RKN4 step (63 on the default 64 x 8 tiles of 16 planes, where 8
+ *  workgroups walk 16 planes each), 128^3 80 us (95); levels from 130^3 up
  *  have a rule of their own below. */
 inline LaunchCfg LaunchRule::pick(int fused) const {
     LaunchCfg c;
@@ -239,7 +239,7 @@ inline LaunchCfg LaunchRule::pick(int fused) const {
         // 3: 144 us against 116 at 160^3, 575 against 492 at 300^3).
         // Automatic chunks give every kernel four rounds or more.  Two rows
         // per thread for one field at radius 1 or in leapfrog from 200^3 up
-        // (172 against 181 us, 105 against 113, equal from 256^3), else 8
+        // (138 against 156 us, 104 against 112, equal from 256^3), else 8
         // wavefronts.
         c.tz = 0;
         const bool two = nfields == 1 && (R == 1 || integrator == 11) &&
